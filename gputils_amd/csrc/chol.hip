@@ -29,6 +29,7 @@
 #include "chol_mixed.hpp"
 #include "chol_small.hpp"
 #include "common.hpp"
+#include "householder.hpp"
 
 namespace gputils {
 namespace chol {
@@ -487,9 +488,354 @@ __global__ __launch_bounds__(kThreads) void posv_kernel(int n, int nrhs, T *A, i
     }
 }
 
+// ------------------------------------------------- larger n, one workgroup --
+// n in (128, kStripMaxN]: the block triangle no longer fits the LDS, so L
+// stays in global memory (one matrix is a few hundred KB: L2 resident) and
+// the factorisation is left-looking by block columns of 16.  Eight
+// wavefronts: wave 0 factors the diagonal blocks, the others own the
+// 16-row strips I = (wave - 1) + 7 s.  What bounds it is the chain of
+// diagonal blocks (16 dependent pivots each), so everything else runs
+// beside it: while wave 0 factors block J, the strips finish column J with
+// the block product of column J - 1 and form column J + 1 up to K = J - 1
+// from L in global memory.  Two barriers per block column, no trailing
+// matrix is written back.  A strip's column is kept transposed (lane % 16 =
+// row, items = columns): that is the accumulator layout of
+// D[j][i] = sum_k L_J[j][k] L_I[i][k], it is a B operand for the next
+// product without any data movement, and its loads and stores are
+// contiguous down a column.
+// 256 systems of n = 200 in FP64, factorisation: the unblocked kernel that
+// read and wrote the whole trailing matrix for each column took 3424 us,
+// this one 73 us.
+constexpr int kStripThreads = 512;
+constexpr int kStripWorkers = kStripThreads / kWave - 1;
+constexpr int kStripSlots = 6;  // strips per wavefront: more spill the FP64 accumulators
+constexpr int64_t kStripMaxN = 16 * kStripWorkers * kStripSlots;
+static_assert(kStripMaxN <= 2 * kStripThreads, "potrs_strips_kernel holds two rows a thread");
+constexpr int64_t kStripMaxLd = 1 << 26;  // lane offsets of up to 13 columns are 32-bit
+
+template <typename T, int S>
+__global__ __launch_bounds__(kStripThreads) void potrf_strips_kernel(int n, T *A, int64_t lda, int64_t strideA,
+                                                                     int *info, int64_t batch) {
+    using M = Mfma16<T>;
+    __shared__ T dg[2][256];  // diagonal block J, then its inverse (slot J & 1)
+    __shared__ T lo[256];     // L_{J+1,J}
+    __shared__ int s_flag;
+    const int64_t b = blockIdx.x;
+    if (b >= batch) return;
+    T *a = A + b * strideA;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave - 1;
+    const int c = lane & 15;
+    const int nb = (n + 15) >> 4;
+    if (threadIdx.x < 256) {
+        const int i = threadIdx.x & 15, k = threadIdx.x >> 4;
+        dg[0][sw(i, k)] = (i >= k) ? a[i + (int64_t)k * lda] : T(0);  // n > 16
+    }
+    if (wave == 0) {
+        // the diagonal chain; its barriers pair with the workers' below
+        __syncthreads();
+        int fail = 0;
+#pragma unroll 1
+        for (int J = 0; J < nb; ++J) {
+            const int f = factor_diag_block(dg[J & 1], a + 16 * J + (int64_t)16 * J * lda, lda, n - 16 * J);
+            fail = (f >= 0) ? 16 * J + f + 1 : 0;  // uniform
+            if (lane == 0) s_flag = fail;
+            __syncthreads();
+            if (fail != 0 || J + 1 == nb) break;
+            __syncthreads();
+        }
+        if (lane == 0 && info != nullptr) info[b] = fail;
+        return;
+    }
+    typename M::acc_t acc[S], nxt[S], lr[S];  // column J, column J + 1 so far, L_{I,J-1}
+    // Step t of a 16x16 block takes column drow(lane, t) = drow(lane, 0) +
+    // drow(0, t) of it: uniform column pointers plus one 32-bit lane offset
+    // per strip (its row, clamped into the matrix: what a lane past n
+    // computes stays in its own row and is not stored).
+    unsigned rs[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        acc[s] = nxt[s] = lr[s] = M::zero();
+        const int r = 16 * (w + kStripWorkers * s) + c;
+        rs[s] = (unsigned)((r < n ? r : n - 1) + M::drow(lane, 0) * (int)lda);
+    }
+    // A_{I,J}: slots past their strips' turn load and compute too, so that
+    // no branch splits the accumulators; nothing of theirs is used.  Entries
+    // above the diagonal of A_{J,J} stay above it.  The last block column
+    // (only its diagonal block is left) must not be read past column n.
+    auto load_block = [&](int s, int J) {
+        typename M::acc_t v;
+        const T *p = a + (int64_t)16 * J * lda;
+        if (J + 1 < nb) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) v[t] = (p + M::drow(0, t) * lda)[rs[s]];
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                v[t] = (16 * J + M::drow(lane, t) < n) ? (p + M::drow(0, t) * lda)[rs[s]] : T(0);
+        }
+        return v;
+    };
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc[s] = load_block(s, 0);
+    __syncthreads();
+#pragma unroll 1
+    for (int J = 0; J < nb; ++J) {
+        if (J > 0) {
+            T lj[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) lj[t] = -lo[sw(c, M::drow(lane, t))];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int s = 0; s < S; ++s) acc[s] = M::fma(lj[t], lr[s][t], acc[s]);
+        }
+        if (J + 1 < nb) {
+            // column J + 1 over K < J
+#pragma unroll
+            for (int s = 0; s < S; ++s) nxt[s] = load_block(s, J + 1);
+            const int rj = 16 * (J + 1) + c;
+            const unsigned pj = (unsigned)((rj < n ? rj : n - 1) + M::drow(lane, 0) * (int)lda);
+            // the strips still below column J + 1 are the slots from
+            // `first` on: one loop for each, without branches inside
+            auto sum_columns = [&](auto first_c) {
+                constexpr int first = decltype(first_c)::value;
+                const T *ak = a;
+#pragma unroll 1
+                for (int K = 0; K < J; ++K, ak += 16 * lda) {
+                    T x[4], y[S][4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) x[t] = -(ak + M::drow(0, t) * lda)[pj];
+#pragma unroll
+                    for (int s = first; s < S; ++s)
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) y[s][t] = (ak + M::drow(0, t) * lda)[rs[s]];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int s = first; s < S; ++s) nxt[s] = M::fma(x[t], y[s][t], nxt[s]);
+                }
+            };
+            const int first = (J - w) < 0 ? 0 : (J - w) / kStripWorkers + 1;  // S or more: none left here
+            if (first == 0) sum_columns(std::integral_constant<int, 0>());
+            else if (first == 1) sum_columns(std::integral_constant<int, 1>());
+            if constexpr (S > 2) {
+                if (first == 2) sum_columns(std::integral_constant<int, 2>());
+                else if (first == 3) sum_columns(std::integral_constant<int, 3>());
+            }
+            if constexpr (S > 4) {
+                if (first == 4) sum_columns(std::integral_constant<int, 4>());
+                else if (first == 5) sum_columns(std::integral_constant<int, 5>());
+            }
+        }
+        __syncthreads();
+        if (s_flag != 0 || J + 1 == nb) break;  // uniform
+        const T *D = dg[J & 1];
+        T d[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) d[t] = D[sw(c, M::drow(lane, t))];
+        T *pl = a + (int64_t)16 * J * lda;
+#pragma unroll
+        for (int s = 0; s < S; ++s) lr[s] = M::zero();
+        // L_IJ^T = D_J (A_IJ - ...)^T
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int s = 0; s < S; ++s) lr[s] = M::fma(d[t], acc[s][t], lr[s]);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int I = w + kStripWorkers * s;
+            if (I == J + 1) {
+                typename M::acc_t q = nxt[s];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) q = M::fma(-lr[s][t], lr[s][t], q);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int j = M::drow(lane, t), gi = 16 * I + c, gk = 16 * I + j;
+                    lo[sw(c, j)] = lr[s][t];
+                    dg[(J + 1) & 1][sw(c, j)] = (gi < n && gk < n) ? q[t] : ((c == j) ? T(1) : T(0));
+                }
+            }
+            if (I > J && 16 * I + c < n) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) (pl + M::drow(0, t) * lda)[rs[s]] = lr[s][t];
+            }
+            acc[s] = nxt[s];
+        }
+        __syncthreads();
+    }
+}
+
+// Solve with the factor of a larger matrix (n in (128, kStripMaxN]) for any
+// nrhs, four right-hand sides per pass.  The reference substitution is a
+// chain of 2 n dependent steps; here the diagonal blocks are inverted first
+// (all at once, one wavefront each), so a pass is a chain of 2 n / 16
+// block steps.  Forward: the thread that owns row i keeps its four values
+// in registers and subtracts block column J (its 16 entries of L loaded a
+// step ahead); the wavefront that owns the next block row then multiplies
+// it by its inverse, one barrier per step.  Backward: wavefront w forms the
+// dot products of columns 2 w and 2 w + 1 of block J with the solution below
+// (rows along the lanes, so L is read contiguously), two barriers per step.
+// 256 systems of n = 200 in FP64, one right-hand side: 310 us for the
+// substitution by columns with two barriers and a tree reduction each,
+// 51 us now.
+// skip != nullptr: systems with skip[b] != 0 (a failed factorisation) are
+// left as they are, as LAPACK dposv leaves B.
+// ROWS: rows of a thread, n <= ROWS * kStripThreads.
+template <typename T, int ROWS>
+__global__ __launch_bounds__(kStripThreads) void potrs_strips_kernel(int n, int nrhs, const T *L, int64_t lda,
+                                                                     int64_t strideL, T *B, int64_t ldb,
+                                                                     int64_t strideB, int *info, int64_t batch,
+                                                                     const int *skip) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_strips[];
+    const int64_t b = blockIdx.x;
+    if (b >= batch) return;
+    if (skip != nullptr && skip[b] != 0) return;
+    constexpr int kStripWaves = kStripThreads / kWave;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int nb = (n + 15) >> 4, npad = 16 * nb;
+    T *D = reinterpret_cast<T *>(dyn_strips);  // nb inverses of 16x16 (sw order)
+    T *Y = D + 256 * nb;                       // npad x 4
+    T *Z = Y + npad * kRhsChunk;               // 16 x 4 sums of the backward step
+    const T *l = L + b * strideL;
+    for (int J = wave; J < nb; J += kStripWaves) {
+        T row[16], invd[16], x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int gi = 16 * J + c, gk = 16 * J + k;
+            row[k] = (gi < n && c >= k) ? l[gi + (int64_t)gk * lda] : ((c == k) ? T(1) : T(0));
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) invd[r] = T(1) / readlane(row[r], r);
+        tri_inverse_cols(row, invd, x);
+        if (lane < 16) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) D[256 * J + sw(r, lane)] = x[r];
+        }
+    }
+    T *bb = B + b * strideB;
+    for (int r0 = 0; r0 < nrhs; r0 += kRhsChunk) {
+        __syncthreads();
+        for (int e = threadIdx.x; e < npad * kRhsChunk; e += kStripThreads) {
+            const int row = e % npad, col = e / npad;
+            Y[e] = (row < n && r0 + col < nrhs) ? bb[row + (int64_t)(r0 + col) * ldb] : T(0);
+        }
+        __syncthreads();
+        // forward: this thread's rows and their entries of block column 0
+        T x[ROWS][kRhsChunk], lc[ROWS][16];
+        auto load_col = [&](int J) {
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                const int i = threadIdx.x + kStripThreads * u;
+                if (i >= 16 * (J + 1) && i < n) {
+#pragma unroll
+                    for (int k = 0; k < 16; ++k) lc[u][k] = l[i + (int64_t)(16 * J + k) * lda];
+                }
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) {
+            const int i = threadIdx.x + kStripThreads * u;
+#pragma unroll
+            for (int r = 0; r < kRhsChunk; ++r) x[u][r] = (i < n) ? Y[i + npad * r] : T(0);
+        }
+        load_col(0);
+        if (wave == 0) {
+            const T v = dot16<false>(D, c, Y + npad * g);
+            Y[c + npad * g] = v;
+        }
+        __syncthreads();
+        for (int J = 0; J + 1 < nb; ++J) {
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                const int i = threadIdx.x + kStripThreads * u;
+                if (i >= 16 * (J + 1) && i < n) {
+#pragma unroll
+                    for (int r = 0; r < kRhsChunk; ++r) {
+                        const T *y = Y + 16 * J + npad * r;
+                        T s0 = T(0), s1 = T(0);
+#pragma unroll
+                        for (int k = 0; k < 16; k += 2) {
+                            s0 += lc[u][k] * y[k];
+                            s1 += lc[u][k + 1] * y[k + 1];
+                        }
+                        x[u][r] -= s0 + s1;
+                    }
+                    // the next block row goes through its inverse below
+                    if (i < 16 * (J + 2)) {
+#pragma unroll
+                        for (int r = 0; r < kRhsChunk; ++r) Y[i + npad * r] = x[u][r];
+                    }
+                }
+            }
+            if (J + 2 < nb) load_col(J + 1);
+            if (wave == (((J + 1) >> 2) & (kStripWaves - 1))) {  // holds rows 16 (J + 1) ..
+                hh::wave_sync();
+                T *y = Y + 16 * (J + 1) + npad * g;
+                const T v = dot16<false>(D + 256 * (J + 1), c, y);
+                hh::wave_sync();
+                y[c] = v;
+            }
+            __syncthreads();
+        }
+        // backward
+        for (int J = nb - 1; J >= 0; --J) {
+            if (J + 1 < nb) {
+                T s[2][kRhsChunk];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int r = 0; r < kRhsChunk; ++r) s[q][r] = T(0);
+                for (int i = 16 * (J + 1) + lane; i < n; i += kWave) {
+                    T lv[2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) lv[q] = l[i + (int64_t)(16 * J + 2 * wave + q) * lda];
+#pragma unroll
+                    for (int r = 0; r < kRhsChunk; ++r) {
+                        const T y = Y[i + npad * r];
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) s[q][r] += lv[q] * y;
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int r = 0; r < kRhsChunk; ++r) s[q][r] = wave_sum(s[q][r]);
+                if (lane == 0) {
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int r = 0; r < kRhsChunk; ++r) Z[2 * wave + q + 16 * r] = s[q][r];
+                }
+                __syncthreads();
+            }
+            if (wave == 0) {
+                T *y = Y + 16 * J + npad * g;
+                T v[16];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) v[k] = y[k] - ((J + 1 < nb) ? Z[k + 16 * g] : T(0));
+                T s0 = T(0), s1 = T(0);
+#pragma unroll
+                for (int k = 0; k < 16; k += 2) {
+                    s0 += D[256 * J + sw(k, c)] * v[k];
+                    s1 += D[256 * J + sw(k + 1, c)] * v[k + 1];
+                }
+                hh::wave_sync();
+                y[c] = s0 + s1;
+            }
+            __syncthreads();
+        }
+        for (int e = threadIdx.x; e < npad * kRhsChunk; e += kStripThreads) {
+            const int row = e % npad, col = e / npad;
+            if (row < n && r0 + col < nrhs) bb[row + (int64_t)(r0 + col) * ldb] = Y[e];
+        }
+    }
+    if (threadIdx.x == 0 && info != nullptr) info[b] = 0;
+}
+
 // ----------------------------------------------- large-n global kernels --
-// Correctness path for n > 128: unblocked right-looking algorithm on the
-// matrix in global memory, one workgroup per matrix.
+// Correctness path for what the strips do not take: unblocked right-looking algorithm on
+// the matrix in global memory, one workgroup per matrix.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void potrf_global_kernel(int n, T *A, int64_t lda,
                                                                 int64_t strideA, int *info,
@@ -521,14 +867,13 @@ __global__ __launch_bounds__(kThreads) void potrf_global_kernel(int n, T *A, int
     if (threadIdx.x == 0 && info != nullptr) info[b] = s_fail;
 }
 
-// skip != nullptr: systems with skip[b] != 0 (a failed factorisation) are
-// left as they are, as LAPACK dposv leaves B.
+// skip as in potrs_strips_kernel.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void potrs_global_kernel(int n, int nrhs, const T *L,
                                                                 int64_t lda, int64_t strideL, T *B,
                                                                 int64_t ldb, int64_t strideB,
                                                                 int *info, int64_t batch,
-                                                                const int *skip = nullptr) {
+                                                                const int *skip) {
     const int64_t b = blockIdx.x;
     if (b >= batch) return;
     if (skip != nullptr && skip[b] != 0) return;
@@ -587,8 +932,36 @@ int potrf_dispatch(int64_t n, T *A, int64_t lda, int64_t strideA, int *info, int
     if (n <= 48) hipLaunchKernelGGL((potrf_kernel<T, 3>), grid, block, 0, st, (int)n, A, lda, strideA, info, batch);
     else if (n <= 64) hipLaunchKernelGGL((potrf_kernel<T, 4>), grid, block, 0, st, (int)n, A, lda, strideA, info, batch);
     else if (n <= 128) hipLaunchKernelGGL((potrf_kernel<T, 8>), grid, block, 0, st, (int)n, A, lda, strideA, info, batch);
-    else hipLaunchKernelGGL((potrf_global_kernel<T>), grid, block, 0, st, (int)n, A, lda, strideA, info, batch);
+    else if (lda > kStripMaxLd || n > kStripMaxN)
+        hipLaunchKernelGGL((potrf_global_kernel<T>), grid, block, 0, st, (int)n, A, lda, strideA, info, batch);
+    else if (n <= 16 * kStripWorkers * 2)
+        hipLaunchKernelGGL((potrf_strips_kernel<T, 2>), grid, dim3(kStripThreads), 0, st, (int)n, A, lda, strideA, info, batch);
+    else if (n <= 16 * kStripWorkers * 4)
+        hipLaunchKernelGGL((potrf_strips_kernel<T, 4>), grid, dim3(kStripThreads), 0, st, (int)n, A, lda, strideA, info, batch);
+    else
+        hipLaunchKernelGGL((potrf_strips_kernel<T, kStripSlots>), grid, dim3(kStripThreads), 0, st, (int)n, A, lda, strideA, info, batch);
     return launch_check("potrf_kernel");
+}
+
+// The solve for n > 128; skip as in the kernels.
+template <typename T>
+int potrs_large(int64_t n, int64_t nrhs, const T *L, int64_t lda, int64_t strideL, T *B, int64_t ldb,
+                int64_t strideB, int *info, int64_t batch, const int *skip, hipStream_t st) {
+    const int64_t nb = ceil_div(n, 16);
+    if (n <= kStripMaxN) {
+        // at most 108 KB of LDS (n = kStripMaxN in FP64)
+        const size_t lds = sizeof(T) * (size_t)(256 * nb + 16 * nb * kRhsChunk + 16 * kRhsChunk);
+        auto kern = n <= kStripThreads ? potrs_strips_kernel<T, 1> : potrs_strips_kernel<T, 2>;
+        if (lds > 64 * 1024)
+            GPUTILS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3((unsigned)batch), dim3(kStripThreads), lds, st, (int)n, (int)nrhs, L, lda,
+                           strideL, B, ldb, strideB, info, batch, skip);
+        return launch_check("potrs_strips_kernel");
+    }
+    hipLaunchKernelGGL((potrs_global_kernel<T>), dim3((unsigned)batch), dim3(kThreads), 0, st, (int)n, (int)nrhs, L,
+                       lda, strideL, B, ldb, strideB, info, batch, skip);
+    return launch_check("potrs_global_kernel");
 }
 
 template <typename T>
@@ -603,7 +976,7 @@ int potrs_dispatch(int64_t n, int64_t nrhs, const T *L, int64_t lda, int64_t str
     if (n <= 48) GPUTILS_POTRS(3);
     else if (n <= 64) GPUTILS_POTRS(4);
     else if (n <= 128) GPUTILS_POTRS(8);
-    else hipLaunchKernelGGL((potrs_global_kernel<T>), grid, block, 0, st, (int)n, (int)nrhs, L, lda, strideL, B, ldb, strideB, info, batch);
+    else return potrs_large<T>(n, nrhs, L, lda, strideL, B, ldb, strideB, info, batch, nullptr, st);
 #undef GPUTILS_POTRS
     return launch_check("potrs_kernel");
 }
@@ -706,9 +1079,7 @@ int gputils_dposv_batched(int64_t n, int64_t nrhs, double *A, int64_t lda, int64
         GPUTILS_ARG(info != nullptr, 9, "info is NULL (needed for n > 128)");
         const int rc = chol::potrf_dispatch<double>(n, A, lda, strideA, info, batch, st);
         if (rc != GPUTILS_OK || nrhs == 0) return rc;
-        hipLaunchKernelGGL((chol::potrs_global_kernel<double>), dim3((unsigned)batch), dim3(chol::kThreads), 0, st,
-                           (int)n, (int)nrhs, A, lda, strideA, B, ldb, strideB, (int *)nullptr, batch, info);
-        return launch_check("potrs_global_kernel");
+        return chol::potrs_large<double>(n, nrhs, A, lda, strideA, B, ldb, strideB, nullptr, batch, info, st);
     }
     return chol::posv_dispatch<double, true>(n, nrhs, A, lda, strideA, B, ldb, strideB, B, ldb,
                                              strideB, info, batch, nullptr, st);
