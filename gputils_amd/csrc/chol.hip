@@ -89,15 +89,17 @@ __device__ __forceinline__ void store_offdiag(T *__restrict__ A, int64_t lda, in
     }
 }
 
-// Pivot of column k: s = sqrt(d) and inv = 1/s, for d > 0.  FP32 uses the
-// hardware reciprocal square root (v_rsq_f32, 1 ulp).  FP64 refines the
-// hardware estimate v_rsq_f64 instead of running the IEEE square root and
-// divide sequences (about 30 dependent operations on the critical path of
-// every column): one coupled Goldschmidt step for sqrt(d) and 1/(2 sqrt(d)),
-// then one Newton correction of each.  s comes out correctly rounded and
-// inv within 1.5 ulp of 1/sqrt(d) (an estimate error up to 2^-22 checked
-// against exact arithmetic).  Pivots below 2^-767 are scaled by 2^256
-// first, as the library square root does, to keep the estimate accurate.
+// Pivot of column k: inv = 1/sqrt(d), and s = sqrt(d), for d > 0.  inv is on
+// the critical path of every column, s is not.  FP32 uses the hardware
+// reciprocal square root (v_rsq_f32, 1 ulp).  FP64 refines the hardware
+// estimate r = v_rsq_f64: with e = 1 - d r^2 (one rounding of d r), one third
+// order step inv = r + r e (1/2 + 3/8 e) leaves the estimate's error cubed
+// (2^-22 or better becomes below 2^-63): inv is within 1 ulp and s, d inv with
+// one Newton correction (d - s^2) inv / 2, is correctly rounded (60000
+// pivots with estimate errors up to 2^-22 against exact arithmetic).  Five dependent
+// operations behind the estimate instead of the eight of two coupled steps.
+// Pivots below 2^-767 are scaled by 2^256 first, as the library square root
+// does, to keep the estimate accurate.
 __device__ __forceinline__ void pivot(float d, float &s, float &inv) {
     inv = __builtin_amdgcn_rsqf(d);
     s = d * inv;
@@ -106,34 +108,122 @@ __device__ __forceinline__ void pivot(double d, double &s, double &inv) {
     const bool tiny = d < 0x1p-767;
     const double dd = tiny ? d * 0x1p+256 : d;
     const double r = __builtin_amdgcn_rsq(dd);
-    double g = dd * r, h = 0.5 * r;
-    double e = __builtin_fma(-g, h, 0.5);
-    g = __builtin_fma(g, e, g);
-    h = __builtin_fma(h, e, h);
-    e = __builtin_fma(-g, g, dd);
-    g = __builtin_fma(e, h, g);
-    double q = h + h;
-    e = __builtin_fma(-g, q, 1.0);
-    q = __builtin_fma(q, e, q);
+    const double e = __builtin_fma(-(dd * r), r, 1.0);
+    const double q = __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
+    double g = dd * q;
+    g = __builtin_fma(__builtin_fma(-g, g, dd), 0.5 * q, g);
     s = tiny ? g * 0x1p-128 : g;
     inv = tiny ? q * 0x1p+128 : q;
 }
 
-// In registers of one wavefront (lane r < 16 holds row r of the block),
-// invert the lower triangular L (row[]) given the reciprocals of its
-// diagonal (uniform): lane c returns column c of L^{-1} in x[].
-template <typename T>
-__device__ __forceinline__ void tri_inverse_cols(const T (&row)[16], const T (&invd)[16], T (&x)[16]) {
-    const int lane = threadIdx.x & 63;
+// d += (v of lane LANE of the 16-lane row) * w: the FMA takes the other
+// lane's value by DPP (row_newbcast, the control that 64-bit arithmetic
+// takes), where readlane and an FMA would be three instructions in FP64.
+// The compiler does not form it by itself and does not see the hazards
+// inside, so every group of them starts with the two wait states that a DPP
+// source needs after a VALU write and ends with the one that a readlane of
+// its result needs.
+template <int LANE>
+__device__ __forceinline__ void fma_lane(double &d, double v, double w) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 0" : "+v"(d) : "v"(v), "v"(w), "n"(LANE));
+}
+// FP32 is faster with readlane: two instructions, no wait states
+// (v_fmac_f32_dpp made a 16x16 block 4096 cycles instead of 3701).
+template <int LANE>
+__device__ __forceinline__ void fma_lane(float &d, float v, float w) {
+    d = fmaf(readlane(v, LANE), w, d);
+}
+// d_i += (v of lane LANE + i) * w, i < 4
+template <int LANE>
+__device__ __forceinline__ void fma_lanes4(double &d0, double &d1, double &d2, double &d3, double v, double w) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\ts_nop 0"
+        : "+v"(d0), "+v"(d1), "+v"(d2), "+v"(d3)
+        : "v"(v), "v"(w), "n"(LANE), "n"(LANE + 1), "n"(LANE + 2), "n"(LANE + 3));
+}
+template <int LANE>
+__device__ __forceinline__ void fma_lanes4(float &d0, float &d1, float &d2, float &d3, float v, float w) {
+    fma_lane<LANE>(d0, v, w);
+    fma_lane<LANE + 1>(d1, v, w);
+    fma_lane<LANE + 2>(d2, v, w);
+    fma_lane<LANE + 3>(d3, v, w);
+}
+// acc0, acc1 += v_p(lane LANE) w_p for p, p + 1, p + 2, p + 3 (two chains)
+template <int LANE, typename T>
+__device__ __forceinline__ void dot_lane4(T &acc0, T &acc1, T v0, T v1, T v2, T v3, T w0, T w1, T w2, T w3) {
+    if constexpr (sizeof(T) == 8)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %2, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %3, %7 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %0, %4, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %5, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf"
+            : "+v"(acc0), "+v"(acc1)
+            : "v"(v0), "v"(v1), "v"(v2), "v"(v3), "v"(w0), "v"(w1), "v"(w2), "v"(w3), "n"(LANE));
+    else {
+        fma_lane<LANE>(acc0, v0, w0);
+        fma_lane<LANE>(acc1, v1, w1);
+        fma_lane<LANE>(acc0, v2, w2);
+        fma_lane<LANE>(acc1, v3, w3);
+    }
+}
+
+// Row K of L^{-1} (lane c holding column c), without the division by the
+// diagonal: e_K - sum_{p<K} L(K, p) x[p], from nx[p] = -x[p]; row[] holds
+// the rows of L, lane r its row r, in every 16-lane row.
+template <int K, typename T>
+__device__ __forceinline__ T inverse_row(const T (&row)[16], const T (&nx)[16]) {
+    T a0 = ((int)(threadIdx.x & 15) == K) ? T(1) : T(0), a1 = T(0);
+    constexpr int K4 = K & ~3;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        T acc = (lane == r) ? T(1) : T(0);
+    for (int p = 0; p < K4; p += 4)
+        dot_lane4<K>(a0, a1, row[p], row[p + 1], row[p + 2], row[p + 3], nx[p], nx[p + 1], nx[p + 2], nx[p + 3]);
 #pragma unroll
-        for (int p = 0; p < r; ++p) acc -= readlane(row[p], r) * x[p];
-        x[r] = acc * invd[r];
-        // x[r] is computed here: left to the compiler, every row's readlane
-        // results were hoisted into SGPRs and spilled (about 450 spills)
-        asm volatile("" : "+v"(x[r]));
+    for (int p = K4; p < K; ++p) {
+        if (p & 1) fma_lane<K>(a1, row[p], nx[p]);
+        else fma_lane<K>(a0, row[p], nx[p]);
+    }
+    return a0 + a1;
+}
+
+// Steps K.. of the inversion of a lower triangular L (row[] as above), dinv
+// the reciprocal of the lane's own diagonal entry: nx[K] = -row K of L^{-1}.
+template <int K, typename T>
+__device__ __forceinline__ void tri_inverse_steps(const T (&row)[16], T dinv, T (&nx)[16]) {
+    if constexpr (K < 16) {
+        nx[K] = -inverse_row<K>(row, nx) * readlane(dinv, K);
+        asm volatile("" : "+v"(nx[K]));  // as in factor_steps
+        tri_inverse_steps<K + 1>(row, dinv, nx);
+    }
+}
+
+// Steps K.. of the factorisation of a 16x16 block (see factor_diag_block).
+template <int K, typename T>
+__device__ __forceinline__ void factor_steps(T (&row)[16], T (&nx)[16], int lane, int &fail) {
+    if constexpr (K < 16) {
+        const T d = readlane(row[K], K);
+        if (fail < 0 && !(d > T(0))) fail = K;  // uniform; also catches NaN
+        T sq, inv;
+        pivot(d, sq, inv);
+        const T lk = ((lane & 15) == K) ? sq : row[K] * inv;
+        row[K] = lk;
+        const T nl = -lk;
+        constexpr int J4 = K + 1 + ((15 - K) & 3);  // the first 0..3 columns singly, the rest by fours
+        if constexpr (K < 15) {
+            if constexpr (J4 > K + 1) fma_lane<K + 1>(row[K + 1], lk, nl);
+            if constexpr (J4 > K + 2) fma_lane<K + 2>(row[K + 2], lk, nl);
+            if constexpr (J4 > K + 3) fma_lane<K + 3>(row[K + 3], lk, nl);
+            if constexpr (J4 < 16) fma_lanes4<J4>(row[J4], row[J4 + 1], row[J4 + 2], row[J4 + 3], lk, nl);
+            if constexpr (J4 + 4 < 16) fma_lanes4<J4 + 4>(row[J4 + 4], row[J4 + 5], row[J4 + 6], row[J4 + 7], lk, nl);
+            if constexpr (J4 + 8 < 16) fma_lanes4<J4 + 8>(row[J4 + 8], row[J4 + 9], row[J4 + 10], row[J4 + 11], lk, nl);
+        }
+        nx[K] = -inverse_row<K>(row, nx) * inv;
+        // left to the compiler, every row's readlane results were hoisted
+        // into SGPRs and spilled
+        asm volatile("" : "+v"(nx[K]));
+        factor_steps<K + 1>(row, nx, lane, fail);
     }
 }
 
@@ -142,14 +232,18 @@ __device__ __forceinline__ void tri_inverse_cols(const T (&row)[16], const T (&i
 // the factor L itself is written there (rows/cols < nvalid).
 // Returns the index (0..15) of the first non-positive pivot or -1.
 //
-// Lane r < 16 holds row r.  Step k scales column k, applies its rank-1
-// update to the columns right of it and forms row k of L^{-1} (lane c
-// holding column c), whose inputs -- row k of L -- are final at that
-// point.  The 16 steps have no branch between them (a failed pivot is only
-// recorded; the NaNs it spreads are never stored), so the scheduler can
-// start the pivot of column k + 1 as soon as its own update is done and
-// overlap it with the rest of step k.  Entries above the diagonal are
-// updated with garbage and never read: only lanes r > j read row[j].
+// Lane r < 16 holds row r (the other 16-lane rows repeat it).  Step k
+// scales column k, applies its rank-1 update to the columns right of it and
+// forms row k of L^{-1} (lane c holding column c), whose inputs -- row k of
+// L -- are final at that point.  What bounds it is one wavefront's chain of
+// pivots and its 240 FMAs, each taking its broadcast operand by DPP (about
+// 9 cycles each; readlane and FMA: 12).  2048 FP64 systems of n = 128:
+// factorisation 213 -> 205 us, solve (whose inverses now divide once per
+// block instead of once per row) 99 -> 92 us, both fused 274 -> 260 us.  The 16 steps
+// have no branch between them (a failed pivot is only recorded; the NaNs it
+// spreads are never stored), so the pivot chain of column k + 1 overlaps
+// the rest of step k.  Entries above the diagonal are updated with garbage
+// and never read: only lanes r > j read row[j].
 template <typename T>
 __device__ __forceinline__ int factor_diag_block(T *blk, T *Lout, int64_t ldo, int nvalid) {
     // a lane index the compiler cannot relate to the one of the other
@@ -157,29 +251,11 @@ __device__ __forceinline__ int factor_diag_block(T *blk, T *Lout, int64_t ldo, i
     // used instead of being kept live in SGPRs across the kernel
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
-    T row[16], x[16];
+    T row[16], nx[16];
 #pragma unroll
     for (int c = 0; c < 16; ++c) row[c] = blk[sw(lane & 15, c)];
     int fail = -1;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const T d = readlane(row[k], k);
-        if (fail < 0 && !(d > T(0))) fail = k;  // uniform; also catches NaN
-        T sq, inv;
-        pivot(d, sq, inv);
-        const T lk = (lane == k) ? sq : row[k] * inv;
-        row[k] = lk;
-#pragma unroll
-        for (int j = k + 1; j < 16; ++j) row[j] -= lk * readlane(lk, j);
-        // row k of L^{-1}: x[k] = (e_k - sum_{p<k} L(k, p) x[p]) / L(k, k)
-        T acc = (lane == k) ? T(1) : T(0);
-#pragma unroll
-        for (int p = 0; p < k; ++p) acc -= readlane(row[p], k) * x[p];
-        x[k] = acc * inv;
-        // left to the compiler, every row's readlane results were hoisted
-        // into SGPRs and spilled
-        asm volatile("" : "+v"(x[k]));
-    }
+    factor_steps<0>(row, nx, lane, fail);
     if (fail >= 0) return fail;
     if (Lout != nullptr && lane < nvalid) {
 #pragma unroll
@@ -188,7 +264,7 @@ __device__ __forceinline__ int factor_diag_block(T *blk, T *Lout, int64_t ldo, i
     }
     if (lane < 16) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) blk[sw(r, lane)] = x[r];
+        for (int r = 0; r < 16; ++r) blk[sw(r, lane)] = -nx[r];
     }
     return -1;
 }
@@ -298,15 +374,13 @@ __device__ __forceinline__ void invert_diag_blocks(T *L, int nb) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int J = wave; J < nb; J += kWaves) {
         T *dJ = L + (tri(J) + J) * 256;
-        T row[16], invd[16], x[16];
+        T row[16], nx[16];
 #pragma unroll
         for (int c = 0; c < 16; ++c) row[c] = dJ[sw(lane & 15, c)];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) invd[r] = T(1) / readlane(row[r], r);
-        tri_inverse_cols(row, invd, x);
+        tri_inverse_steps<0>(row, T(1) / dJ[sw(lane & 15, lane & 15)], nx);
         if (lane < 16) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) dJ[sw(r, lane)] = x[r];
+            for (int r = 0; r < 16; ++r) dJ[sw(r, lane)] = -nx[r];
         }
     }
 }
@@ -390,8 +464,11 @@ __device__ __forceinline__ void solve_blocked(const T *L, int nb, T *Y) {
 
 // ------------------------------------------------------------ kernels --
 // Factor only (API: CholeskyBatchFactoriser::factorise).
+// n <= 64 leaves the LDS for many workgroups: four wavefronts per SIMD are
+// worth a few spilled registers (4096 FP64 systems of n = 40: 118 us with
+// two, 77 us with four).
 template <typename T, int NB>
-__global__ __launch_bounds__(kThreads) void potrf_kernel(int n, T *A, int64_t lda, int64_t strideA,
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NB <= 4 ? 4 : 2))) void potrf_kernel(int n, T *A, int64_t lda, int64_t strideA,
                                                          int *info, int64_t batch) {
     __shared__ T L[tri(NB) * 256];
     __shared__ int s_flag;
@@ -505,7 +582,7 @@ __global__ __launch_bounds__(kThreads) void posv_kernel(int n, int nrhs, T *A, i
 // contiguous down a column.
 // 256 systems of n = 200 in FP64, factorisation: the unblocked kernel that
 // read and wrote the whole trailing matrix for each column took 3424 us,
-// this one 73 us.
+// this one 70 us.
 constexpr int kStripThreads = 512;
 constexpr int kStripWorkers = kStripThreads / kWave - 1;
 constexpr int kStripSlots = 6;  // strips per wavefront: more spill the FP64 accumulators
@@ -677,7 +754,7 @@ __global__ __launch_bounds__(kStripThreads) void potrf_strips_kernel(int n, T *A
 // (rows along the lanes, so L is read contiguously), two barriers per step.
 // 256 systems of n = 200 in FP64, one right-hand side: 310 us for the
 // substitution by columns with two barriers and a tree reduction each,
-// 51 us now.
+// 47 us now.
 // skip != nullptr: systems with skip[b] != 0 (a failed factorisation) are
 // left as they are, as LAPACK dposv leaves B.
 // ROWS: rows of a thread, n <= ROWS * kStripThreads.
@@ -699,18 +776,15 @@ __global__ __launch_bounds__(kStripThreads) void potrs_strips_kernel(int n, int 
     T *Z = Y + npad * kRhsChunk;               // 16 x 4 sums of the backward step
     const T *l = L + b * strideL;
     for (int J = wave; J < nb; J += kStripWaves) {
-        T row[16], invd[16], x[16];
+        T row[16], nx[16];
+        const int gi = 16 * J + c;
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int gi = 16 * J + c, gk = 16 * J + k;
-            row[k] = (gi < n && c >= k) ? l[gi + (int64_t)gk * lda] : ((c == k) ? T(1) : T(0));
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) invd[r] = T(1) / readlane(row[r], r);
-        tri_inverse_cols(row, invd, x);
+        for (int k = 0; k < 16; ++k)
+            row[k] = (gi < n && c >= k) ? l[gi + (int64_t)(16 * J + k) * lda] : ((c == k) ? T(1) : T(0));
+        tri_inverse_steps<0>(row, (gi < n) ? T(1) / l[gi + (int64_t)gi * lda] : T(1), nx);
         if (lane < 16) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) D[256 * J + sw(r, lane)] = x[r];
+            for (int r = 0; r < 16; ++r) D[256 * J + sw(r, lane)] = -nx[r];
         }
     }
     T *bb = B + b * strideB;
