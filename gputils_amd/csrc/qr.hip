@@ -8,7 +8,9 @@
 // plan: FP32 Householder QR with FP64 norms and dot products plus one FP64
 // refinement step).
 //
-// One 256-thread workgroup per matrix.  The matrix lives in LDS when it
+// Matrices of up to 1024 rows (triangles of up to 512) go to the register
+// kernels of qr_regs.hip.  The uniform kernels here take what is larger: one
+// 256-thread workgroup per matrix.  The matrix lives in LDS when it
 // fits (otherwise the kernel works on it in global memory).  Column c is
 // owned by wavefront c % 4.  Step j: every wave applies reflector j to the
 // columns it owns; the owner of column j+1 does that column first and then
@@ -22,6 +24,7 @@
 
 #include "common.hpp"
 #include "householder.hpp"
+#include "qr_regs.hpp"
 
 namespace gputils {
 namespace qr {
@@ -637,6 +640,8 @@ int launch_ragged(int maxe, int method, int waves, int grid, hipStream_t st, con
 template <typename T>
 int gels_dispatch(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t strideA, T *B,
                   int64_t ldb, int64_t strideB, T *tauws, int *info, int64_t batch, hipStream_t st) {
+    if (m <= qrr::kMaxRows && n <= qrr::kMaxTri)
+        return qrr::gels<T>(m, n, nrhs, A, lda, strideA, B, ldb, strideB, info, batch, st);
     const size_t dyn = sizeof(T) * (size_t)(n + m);
     if (dyn > 48 * 1024) {
         set_error("gels: m + n too large for the vector workspace");
@@ -648,8 +653,7 @@ int gels_dispatch(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t
     hipLaunchKernelGGL((gels_kernel<T, ME>), grid, block, dyn, st, (int)m, (int)n, (int)nrhs, A, lda, strideA, \
                        B, ldb, strideB, tauws, info, batch)
     constexpr int kBig = (int)(56 * 1024 / sizeof(T));
-    if (mn <= 1024) GPUTILS_GELS(1024);
-    else if (mn <= 4096) GPUTILS_GELS(4096);
+    if (mn <= 4096) GPUTILS_GELS(4096);
     else if (mn <= kBig) GPUTILS_GELS(kBig);
     else GPUTILS_GELS(0);
 #undef GPUTILS_GELS
@@ -659,13 +663,13 @@ int gels_dispatch(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t
 template <typename T>
 int geqrf_dispatch(int64_t m, int64_t n, T *A, int64_t lda, int64_t strideA, T *tau, int64_t strideTau,
                    int *info, int64_t batch, hipStream_t st) {
+    if (m <= qrr::kMaxRows) return qrr::geqrf<T>(m, n, A, lda, strideA, tau, strideTau, info, batch, st);
     const dim3 grid((unsigned)batch), block(kThreads);
     const int64_t mn = m * n;
 #define GPUTILS_GEQRF(ME) \
     hipLaunchKernelGGL((geqrf_kernel<T, ME>), grid, block, 0, st, (int)m, (int)n, A, lda, strideA, tau, strideTau, info, batch)
     constexpr int kBig = (int)(56 * 1024 / sizeof(T));
-    if (mn <= 1024) GPUTILS_GEQRF(1024);
-    else if (mn <= 4096) GPUTILS_GEQRF(4096);
+    if (mn <= 4096) GPUTILS_GEQRF(4096);
     else if (mn <= kBig) GPUTILS_GEQRF(kBig);
     else GPUTILS_GEQRF(0);
 #undef GPUTILS_GEQRF
@@ -871,6 +875,9 @@ GPUTILS_GEQRF_ENTRY(gputils_dgeqrf_batched, double)
         GPUTILS_ARG(batch >= 0 && batch <= 0x7fffffff, 13, "batch out of range");                        \
         GPUTILS_ARG(sizeof(T) * (size_t)m * 4 <= 64 * 1024, 2, "m too large");                           \
         if (m == 0 || ncols == 0 || k == 0 || batch == 0) return GPUTILS_OK;                             \
+        if (m <= qrr::kMaxRows)                                                                          \
+            return qrr::ormqr<T>(trans, m, m, ncols, k, A, lda, strideA, tau, strideTau, C, ldc,         \
+                                 strideC, batch, as_stream(stream));                                     \
         hipLaunchKernelGGL((qr::ormqr_kernel<T>), dim3((unsigned)batch), dim3(qr::kThreads),             \
                            sizeof(T) * (size_t)m * qr::kWaves, as_stream(stream), trans, (int)m,         \
                            (int)ncols, (int)k, A, lda, strideA, tau, strideTau, C, ldc, strideC, batch); \
@@ -889,6 +896,8 @@ GPUTILS_ORMQR_ENTRY(gputils_dormqr_batched, double)
         GPUTILS_ARG(batch >= 0 && batch <= 0x7fffffff, 9, "batch out of range");                         \
         GPUTILS_ARG(sizeof(T) * (size_t)n * 4 <= 64 * 1024, 1, "n too large");                           \
         if (n == 0 || nrhs == 0 || batch == 0) return GPUTILS_OK;                                        \
+        if (n <= qrr::kMaxTri)                                                                           \
+            return qrr::trsm_upper<T>(n, nrhs, R, ldr, strideR, B, ldb, strideB, batch, as_stream(stream)); \
         hipLaunchKernelGGL((qr::trsm_upper_kernel<T>), dim3((unsigned)batch), dim3(qr::kThreads),        \
                            sizeof(T) * (size_t)n * qr::kWaves, as_stream(stream), (int)n, (int)nrhs, R,  \
                            ldr, strideR, B, ldb, strideB, batch);                                        \
