@@ -180,36 +180,14 @@ __device__ __forceinline__ T row16_sum(T x) {
 // its 16 lanes.  Four columns then cost one set of row loads and one
 // four-step reduction, where the 64-lane form below pays a six-step
 // reduction per column.
-// KR < 0: any m, nothing held in registers (two passes over the rows, v
-// read with each; for kernels that cannot spare the registers).
 template <typename T, typename DOT, int NW, int KR>
 __device__ __forceinline__ void apply_reflector_cols16(T *A, int64_t lda, int m, int j, T tau, int c0, int n) {
     const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
     const T *v = A + (int64_t)j * lda;
-    if constexpr (KR < 0) {
-        for (int cq = c0; cq < n; cq += 4 * NW) {
-            const int c = cq + NW * g;
-            const bool ok = c < n;
-            T *x = A + (int64_t)(ok ? c : cq) * lda;
-            DOT w = DOT(0);
-#pragma unroll 4
-            for (int i = j + 1 + l16; i < m; i += 16) w += (DOT)v[i] * (DOT)x[i];
-            const T xj = x[j];
-            w = row16_sum(w) + (DOT)xj;
-            const T tw = ok ? (T)((DOT)tau * w) : T(0);
-            if (ok) {
-#pragma unroll 4
-                for (int i = j + 1 + l16; i < m; i += 16) x[i] -= tw * v[i];
-                if (l16 == 0) x[j] = xj - tw;
-            }
-        }
-        return;
-    }
-    constexpr int KRH = KR > 0 ? KR : 1;
     const int kr = (m - j - 1 + 15) >> 4;  // row groups in use (uniform)
-    T vr[KRH];
+    T vr[KR];
 #pragma unroll
-    for (int k = 0; k < KRH; ++k) {
+    for (int k = 0; k < KR; ++k) {
         const int i = j + 1 + l16 + 16 * k;
         vr[k] = T(0);
         if (k < kr) {
@@ -221,10 +199,10 @@ __device__ __forceinline__ void apply_reflector_cols16(T *A, int64_t lda, int m,
         const int c = cq + NW * g;
         const bool ok = c < n;
         T *x = A + (int64_t)(ok ? c : cq) * lda;
-        T xr[KRH];
+        T xr[KR];
         DOT w = DOT(0);
 #pragma unroll
-        for (int k = 0; k < KRH; ++k) {
+        for (int k = 0; k < KR; ++k) {
             xr[k] = T(0);
             if (k < kr) {
                 const int i = j + 1 + l16 + 16 * k;
@@ -236,7 +214,7 @@ __device__ __forceinline__ void apply_reflector_cols16(T *A, int64_t lda, int m,
         w = row16_sum(w) + (DOT)xj;
         const T tw = ok ? (T)((DOT)tau * w) : T(0);
 #pragma unroll
-        for (int k = 0; k < KRH; ++k) {
+        for (int k = 0; k < KR; ++k) {
             if (k < kr) {
                 const int i = j + 1 + l16 + 16 * k;
                 if (ok && i < m) x[i] = xr[k] - tw * vr[k];

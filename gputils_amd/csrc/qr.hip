@@ -442,6 +442,37 @@ __device__ __forceinline__ void trsv_upper_trans_regs(const float *S, int m, int
     if (lane < n) c[lane] = cv;
 }
 
+// Factorisation of [A b] for the ragged solver with the columns in registers
+// (RegQr), into S (column-major, ld m, b as column n) and tau; MLO < m <=
+// LPC * KR.  Columns of up to 128 rows take 16 lanes, taller ones a wavefront:
+// there the reflector's own chain, four times as long in 16 lanes, counts for
+// more than the cheaper reductions (16 K bucket, a column step 2810 cycles in
+// 16 lanes, 2580 in 64; for 65 to 128 rows 1870 against 2100).  Layouts that
+// no system of the bucket can have are left out.
+template <int MAXE, int NW, int LPC, int KR, int MLO>
+__device__ __forceinline__ void ragged_factor(const double *__restrict__ a, const double *__restrict__ bcol, float *S,
+                                              int m, int n, float *vbuf, float *s_tau, float *tau) {
+    constexpr int kMin = MAXE == 2048 ? 0 : MAXE / 2;  // m n > kMin
+    if constexpr (64 * LPC * KR > kMin) {
+        constexpr int kMaxCols = (MAXE / (MLO + 1) < 64 ? MAXE / (MLO + 1) : 64) + 1;
+        constexpr int kStep = NW * (kWave / LPC);
+        using Q = qrr::RegQr<float, double, float, LPC, NW, KR, (kMaxCols + kStep - 1) / kStep>;
+        static_assert(Q::kV <= 1024, "the reflectors share rd's LDS");
+        Q qr;
+#pragma unroll
+        for (int q = 0; q < Q::kSlots; ++q) {
+            const int c = qr.col(q);
+            if (qr.first(q) <= n) qr.load(q, c < n ? a + (int64_t)c * m : bcol, m, c <= n);  // uniform
+            else qr.clear(q);
+            if (q & 1) asm volatile("" ::: "memory");  // two slots' doubles in flight at a time
+        }
+        qr.factor(n, n + 1, vbuf, s_tau, tau);
+#pragma unroll
+        for (int q = 0; q < Q::kSlots; ++q)
+            if (qr.first(q) <= n) qr.store(q, S + qr.col(q) * m, m, qr.col(q) <= n);
+    }
+}
+
 // One bucket of the ragged plan: workgroup w solves the items
 // wstart[w] .. wstart[w+1]-1, a range the plan balanced by estimated cost
 // (longest-processing-time assignment).  Per system: FP32 Householder QR
@@ -455,10 +486,14 @@ __device__ __forceinline__ void trsv_upper_trans_regs(const float *S, int m, int
 // accuracy also for inconsistent systems, where refining x alone stalls at
 // the FP32 level.  x overwrites b[0:n].  Global loads are batched (eight
 // per thread in flight) because one wavefront per SIMD leaves little else
-// to hide their latency.  METHOD selects the factorisation: 0 stages A in
-// LDS and factorises column by column (hqr_factor, lookahead column in
-// registers, one barrier per column; NW = 2, 4, 8 or 16), 1 keeps panels in
-// registers (hqr_panels, one barrier per panel; NW = 8 or 16).  The plan
+// to hide their latency.  METHOD selects the factorisation: 0 keeps the
+// columns in registers, spread over the wavefronts one by one (RegQr, one
+// barrier per column; NW = 2, 4, 8 or 16), 1 keeps panels of them
+// (hqr_panels, one barrier per panel; NW = 8 or 16).  A column step of method
+// 0 is bound by the chain of the reflector (about 1350 cycles for short
+// columns) and for tall ones by issue; with A streamed from LDS for every
+// column it took 3700 to 5300.  4096 systems of the configuration, one
+// refinement step: default shapes 1547 -> 1035 us, tuned 1112 -> 809 us.  The plan
 // picks METHOD, NW and the grid per bucket.  For one METHOD every system's
 // arithmetic is the same for every NW and every item-to-workgroup
 // assignment, so the results are too; the two methods round the FP32
@@ -505,24 +540,17 @@ __global__ __launch_bounds__(NW * kWave) void gels_ragged_kernel(const RaggedIte
             for (int i = threadIdx.x; i < m; i += NT) bd[i] = bb[i];
             hqr_panels<NW>(a, bb, S, m, n, tau);  // FP64 norms, FP32 dots
         } else {
-            const int mn = m * n;
-            int e0 = threadIdx.x;
-            for (; e0 + 7 * NT < mn; e0 += 8 * NT) {
-                double v[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = a[e0 + u * NT];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) S[e0 + u * NT] = (float)v[u];
-            }
-            for (; e0 < mn; e0 += NT) S[e0] = (float)a[e0];
-            for (int i = threadIdx.x; i < m; i += NT) {
-                const double v = bb[i];
-                bd[i] = v;
-                qb[i] = (float)v;
-            }
+            for (int i = threadIdx.x; i < m; i += NT) bd[i] = bb[i];
+            // FP64 norms, FP32 dots; the layout depends on m alone, so a
+            // system's arithmetic is the same for every NW.  A bucket's systems
+            // have MAXE / 2 < m n <= MAXE (the smallest: m n <= MAXE), which
+            // bounds the columns of each layout; rd is free until r0
+            float *vbuf = reinterpret_cast<float *>(rd);
+            if (m <= 64) ragged_factor<MAXE, NW, 16, 4, 0>(a, bb, S, m, n, vbuf, s_tau, tau);
+            else if (m <= 128) ragged_factor<MAXE, NW, 16, 8, 64>(a, bb, S, m, n, vbuf, s_tau, tau);
+            else if (m <= 256) ragged_factor<MAXE, NW, 64, 4, 128>(a, bb, S, m, n, vbuf, s_tau, tau);
+            else ragged_factor<MAXE, NW, 64, 8, 256>(a, bb, S, m, n, vbuf, s_tau, tau);
             __syncthreads();
-            // FP64 norms, FP32 dots; trailing columns updated by 16-lane groups
-            hqr_factor<float, double, float, NW, -1>(S, m, m, n, tau, s_tau, n + 1);
         }
         if (wave == 0) trsv_upper_regs(S, m, n, qb);  // x0 = R^{-1} (Q^T b)[0:n]
         __syncthreads();
@@ -584,9 +612,13 @@ __global__ __launch_bounds__(NW * kWave) void gels_ragged_kernel(const RaggedIte
                 trsv_upper_regs(S, m, n, dx);                                 // dx = R^{-1} (d1 - h)
                 for (int i = lane; i < n; i += kWave) xd[i] += (double)dx[i];
             }
-            if (wave == 1) apply_q_regs(S, m, n, tau, c, false);  // c = dr = Q [h; d2]
-            __syncthreads();
-            for (int i = threadIdx.x; i < m; i += NT) rd[i] += (double)c[i];
+            // c = dr = Q [h; d2] and the new r: only another step reads them
+            // (n reflectors in a chain, a sixth of a system's time)
+            if (s + 1 < steps) {
+                if (wave == 1) apply_q_regs(S, m, n, tau, c, false);
+                __syncthreads();
+                for (int i = threadIdx.x; i < m; i += NT) rd[i] += (double)c[i];
+            }
         }
         __syncthreads();
         for (int i = threadIdx.x; i < n; i += NT) bb[i] = xd[i];

@@ -8,8 +8,8 @@
 // bounds a step now is the chain reflector -> dot product -> update -> next
 // reflector (about 0.6 us in FP32, 1 us in FP64) and, with many matrices,
 // instruction issue.  Before -> now: least squares of 1024 FP32 100 x 30
-// systems 91 -> 34 us, of 8192 402 -> 164 us; QR of one FP64 600 x 150 matrix
-// 6320 -> 249 us, its 150 columns of Q 10357 -> 63 us.
+// systems 91 -> 33 us, of 8192 402 -> 144 us; QR of one FP64 600 x 150 matrix
+// 6320 -> 250 us, its 150 columns of Q 10357 -> 63 us.
 #include <algorithm>
 
 #include "qr_regs.hpp"

@@ -15,6 +15,44 @@ __device__ __forceinline__ T lanes_sum(T v) {
     else return wave_sum(v);
 }
 
+// Sums over the wavefront of up to four values at once: v_permlane32_swap and
+// v_permlane16_swap leave value i's partial sums in 16-lane row i with one
+// addition per pair of values, then four row steps finish all of them; lane
+// 16 i is value i's sum.  10 additions and swaps for four values, where each
+// alone takes 6 steps of two or three instructions.  A value's additions are
+// the same whatever it shares the registers with.
+__device__ __forceinline__ float swap_add32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double swap_add32(double a, double b) {
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
+}
+template <int N, typename T>
+__device__ __forceinline__ void wave_sums(T (&w)[N]) {
+    static_assert(N >= 1 && N <= 4, "at most four values");
+    // rows 0, 1, 2, 3 of the result: values 0, 2, 1, 3
+    const T lo = swap_add32(w[0], w[N > 1 ? 1 : 0]);
+    const T hi = N > 2 ? swap_add32(w[N > 2 ? 2 : 0], w[N > 3 ? 3 : N > 2 ? 2 : 0]) : lo;
+    const T s = hh::row16_sum(swap_add16(lo, hi));
+    constexpr int kLane[4] = {0, 32, 16, 48};
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = readlane(s, kLane[i]);
+}
+
 // The reflector scalars without the square root and divisions of
 // hh::reflector_scalars: they are on the chain of every column (in FP64 two
 // divisions and a square root are about 400 cycles).  FP64: rsq with a
@@ -51,6 +89,7 @@ template <typename T, typename ACC, typename DOT, int LPC, int NW, int KR, int S
 struct RegQr {
     static constexpr int kGroups = kWave / LPC;      // columns of one slot of a wavefront
     static constexpr int kCols = NW * kGroups * SL;  // columns held
+    static constexpr int kSlots = SL;
     static constexpr int kRows = LPC * KR;
     static constexpr int kV = 2 * kRows;  // LDS elements of the reflector buffers
     T x[SL][KR];
@@ -76,6 +115,10 @@ struct RegQr {
 #pragma unroll
         for (int k = 0; k < KR; ++k)
             if (!(ok && l + LPC * k < m)) x[q][k] = T(0);
+    }
+    __device__ __forceinline__ void clear(int q) {
+#pragma unroll
+        for (int k = 0; k < KR; ++k) x[q][k] = T(0);
     }
     __device__ __forceinline__ void store(int q, T *dst, int m, bool ok) const {
 #pragma unroll
@@ -128,30 +171,46 @@ struct RegQr {
     }
 
     // x_q -= (t v . x_q) v for the columns right of column j in slots Q0 ..
-    // SL - 1 but slot `skip` (uniform; SL for none): the slots' dot products,
+    // Q1 - 1 but slot `skip` (uniform; SL for none): the slots' dot products,
     // their reductions and their updates run side by side
-    template <int Q0>
+    template <int Q0, int Q1>
     __device__ __forceinline__ void update(int skip, int j, int ntot, const T (&vr)[KR], T t) {
-        DOT w[SL];
+        DOT w[Q1 - Q0];
 #pragma unroll
-        for (int q = Q0; q < SL; ++q) {
+        for (int q = Q0; q < Q1; ++q) {
             DOT w0 = DOT(0), w1 = DOT(0);
 #pragma unroll
             for (int k = 0; k < KR; k += 2) {
                 w0 = fma((DOT)vr[k], (DOT)x[q][k], w0);
                 if (k + 1 < KR) w1 = fma((DOT)vr[k + 1], (DOT)x[q][k + 1], w1);
             }
-            w[q] = w0 + w1;
+            w[q - Q0] = w0 + w1;
         }
+        if constexpr (LPC == 64) wave_sums(w);
 #pragma unroll
-        for (int q = Q0; q < SL; ++q) w[q] = (DOT)t * lanes_sum<LPC>(w[q]);
+        for (int q = Q0; q < Q1; ++q) w[q - Q0] = (DOT)t * (LPC == 64 ? w[q - Q0] : hh::row16_sum(w[q - Q0]));
 #pragma unroll
-        for (int q = Q0; q < SL; ++q) {
+        for (int q = Q0; q < Q1; ++q) {
             const int c = col(q);
             if (c > j && c < ntot && q != skip) {
 #pragma unroll
-                for (int k = 0; k < KR; ++k) x[q][k] = fma(-(T)w[q], vr[k], x[q][k]);
+                for (int k = 0; k < KR; ++k) x[q][k] = fma(-(T)w[q - Q0], vr[k], x[q][k]);
             }
+        }
+    }
+    // the same for all slots but those that hold nothing right of column j
+    // (uniform): few slots drop out one by one from the left, many in fours
+    template <int Q0 = 0>
+    __device__ __forceinline__ void update_all(int skip, int j, int ntot, const T (&vr)[KR], T t) {
+        if constexpr (SL <= 3) {
+            if constexpr (Q0 < SL) {
+                if (last(Q0) > j) update<Q0, SL>(skip, j, ntot, vr, t);
+                else update_all<Q0 + 1>(skip, j, ntot, vr, t);
+            }
+        } else if constexpr (Q0 < SL) {
+            constexpr int Q1 = Q0 + 4 < SL ? Q0 + 4 : SL;
+            if (last(Q1 - 1) > j && first(Q0) < ntot) update<Q0, Q1>(skip, j, ntot, vr, t);
+            update_all<Q1>(skip, j, ntot, vr, t);
         }
     }
     // one slot (the owner's next column)
@@ -162,7 +221,10 @@ struct RegQr {
             w0 = fma((DOT)vr[k], (DOT)xc[k], w0);
             if (k + 1 < KR) w1 = fma((DOT)vr[k + 1], (DOT)xc[k + 1], w1);
         }
-        const T tw = (T)((DOT)t * lanes_sum<LPC>(w0 + w1));
+        DOT w[1] = {w0 + w1};
+        if constexpr (LPC == 64) wave_sums(w);
+        else w[0] = hh::row16_sum(w[0]);
+        const T tw = (T)((DOT)t * w[0]);
         if (c > j) {
 #pragma unroll
             for (int k = 0; k < KR; ++k) xc[k] = fma(-tw, vr[k], xc[k]);
@@ -173,36 +235,38 @@ struct RegQr {
     // reflector (a right-hand side ends as Q^T b).  vbuf: kV elements and
     // s_tau two of LDS; tau: n values, LDS or global.  Per column: the
     // reflector is read from LDS, the owner of the next column brings that
-    // one up to date first and forms the next reflector, the others update
-    // what they hold; one barrier.  Ends with a barrier.
+    // one up to date and forms the next reflector, the others update what
+    // they hold; one barrier.  The owner's other columns wait until after the
+    // barrier, off the chain.  Ends with a barrier.
     __device__ __forceinline__ void factor(int n, int ntot, T *vbuf, T *s_tau, T *tau) {
         if (wave == 0) reflect(x[0], 0, vbuf, s_tau, tau);
         __syncthreads();
+        T vr[KR], t = T(0);
+        int late = SL;  // slot formed in the last step: the others wait for its reflector's update
+#pragma unroll
+        for (int k = 0; k < KR; ++k) vr[k] = T(0);
 #pragma unroll 1
         for (int j = 0; j < n; ++j) {
+            if (late < SL) {  // uniform; vr and t are still the last step's
+                update_all(late, j - 1, ntot, vr, t);
+                late = SL;
+            }
             const T *v = vbuf + (j & 1) * kRows;
-            T vr[KR];
 #pragma unroll
             for (int k = 0; k < KR; ++k) vr[k] = v[l + LPC * k];
-            const T t = s_tau[j & 1];
+            t = s_tau[j & 1];
             const int c1 = j + 1;
-            const bool own = c1 < n && wave == c1 % NW;  // uniform
-            const int q1 = own ? c1 / (NW * kGroups) : SL;
-            if (own) {
+            if (c1 < n && wave == c1 % NW) {  // uniform
+                late = c1 / (NW * kGroups);
 #pragma unroll
                 for (int q = 0; q < SL; ++q)
-                    if (q == q1) {
+                    if (q == late) {
                         update_one(x[q], col(q), j, vr, t);  // columns past ntot hold zeros
                         reflect(x[q], c1, vbuf + (c1 & 1) * kRows, s_tau + (c1 & 1), tau);
                     }
+            } else {
+                update_all(SL, j, ntot, vr, t);
             }
-            // slots whose columns are all factorised drop out from the left
-            constexpr int kQ = SL >= 4 ? SL / 4 : 1;
-            if (last(kQ - 1) > j) update<0>(q1, j, ntot, vr, t);
-            else if (SL > kQ && last(2 * kQ - 1 < SL ? 2 * kQ - 1 : 0) > j) update<kQ < SL ? kQ : 0>(q1, j, ntot, vr, t);
-            else if (SL > 2 * kQ && last(3 * kQ - 1 < SL ? 3 * kQ - 1 : 0) > j)
-                update<2 * kQ < SL ? 2 * kQ : 0>(q1, j, ntot, vr, t);
-            else if (SL > 3 * kQ) update<3 * kQ < SL ? 3 * kQ : 0>(q1, j, ntot, vr, t);
             __syncthreads();
         }
     }

@@ -248,8 +248,8 @@ int gputils_dgels_ragged(gputils_gels_plan_t plan, const double *A, double *B, i
                          void *stream);
 /* Launch shape per bucket.  A plan has one bucket per LDS size class in use
  * (FP32 m*n <= 2048, 4096, 8192, 16384, 32768; largest first), one launch
- * each.  Its shape: the factorisation method (0: A staged in LDS and
- * factorised column by column, one barrier per column; 1: panels of
+ * each.  Its shape: the factorisation method (0: columns in registers, spread
+ * over the wavefronts one by one, one barrier per column; 1: panels of
  * 64 / waves columns held in registers, one barrier per panel), the
  * wavefronts per workgroup (2, 4, 8 or 16 for method 0; 8 or 16 for
  * method 1), the workgroups per CU (the grid is min(systems in the
