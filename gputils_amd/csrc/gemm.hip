@@ -3,15 +3,8 @@
 // Replaces cublas?gemmBatched / ?gemm behind DTensor::addAB and operator*
 // (include/tensor.cuh:1286-1338, 645-650).
 //
-// Tiled path: one 256-thread workgroup computes a 64x64 tile of one C_i.
-// K is staged through LDS in chunks (32 for float, 16 for double) with the
-// k index contiguous for both operands (A tile stored transposed).  Each
-// wavefront owns a 32x32 quadrant = 2x2 MFMA tiles of 16x16:
-//   float, FP32 mode   v_mfma_f32_16x16x4_f32      (exact fp32 products)
-//   float, BF16X3 mode v_mfma_f32_16x16x32_bf16 x3: a = ah + al, b = bh + bl
-//                      (bf16 terms), C += ah bh + ah bl + al bh, fp32 acc.
-//   double             v_mfma_f64_16x16x4_f64
-// The C tile is staged through LDS and written column by column (coalesced).
+// Tiled path (gemm_tiled_kernel): any shape, K through LDS, 2x2 MFMA tiles of
+// 16x16 per wavefront.
 //
 // Per-matrix path (C aliasing B, or very narrow C): one workgroup per
 // matrix stages all of B_i in LDS before any C_i element is written, which
@@ -27,17 +20,6 @@ namespace gemm {
 constexpr int kThreads = 256;
 constexpr int kTM = 64, kTN = 64;
 
-template <typename T>
-struct Cfg;
-template <>
-struct Cfg<float> {
-    static constexpr int TK = 32, S = 36;  // k-chunk, LDS row stride (16-byte aligned rows)
-};
-template <>
-struct Cfg<double> {
-    static constexpr int TK = 16, S = 17;
-};
-
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -50,121 +32,236 @@ __device__ inline void split_bf16(const float *v, bf16x8 &hi, bf16x8 &lo) {
     }
 }
 
-// Stage A[i0:i0+64, k0:k0+TK] as As[i][k] and B[k0:k0+TK, j0:j0+64] as
-// Bs[j][k] (both with row stride S), zero outside the matrix.
-template <typename T>
-__device__ void stage(const T *a, int64_t lda, const T *b, int64_t ldb, int m, int n, int k, int i0,
-                      int j0, int k0, T *As, T *Bs) {
-    constexpr int TK = Cfg<T>::TK, S = Cfg<T>::S;
-    // A: consecutive threads walk down a column (contiguous in memory)
-    for (int e = threadIdx.x; e < kTM * TK; e += kThreads) {
-        const int i = e % kTM, kk = e / kTM;
-        const int gi = i0 + i, gk = k0 + kk;
-        As[i * S + kk] = (gi < m && gk < k) ? a[gi + (int64_t)gk * lda] : T(0);
-    }
-    // B: consecutive threads walk down a column of B (k contiguous)
-    for (int e = threadIdx.x; e < kTN * TK; e += kThreads) {
-        const int kk = e % TK, j = e / TK;
-        const int gk = k0 + kk, gj = j0 + j;
-        Bs[j * S + kk] = (gk < k && gj < n) ? b[gk + (int64_t)gj * ldb] : T(0);
-    }
-}
-
+// General kernel: a workgroup of WV x WV wavefronts computes a tile of one
+// C_i, 32x32 per wavefront = 2x2 MFMA tiles of 16x16:
+//   float, FP32 mode   v_mfma_f32_16x16x4_f32      (exact fp32 products)
+//   float, BF16X3 mode v_mfma_f32_16x16x32_bf16 x3: a = ah + al, b = bh + bl
+//                      (bf16 terms), C += al bh + ah bl + ah bh, fp32 acc.
+//   double             v_mfma_f64_16x16x4_f64
+// K goes through two LDS buffers in chunks of TK, k contiguous for both
+// operands; the next chunk's loads are issued before the current one is
+// multiplied, one barrier per chunk, so a workgroup waits for memory only
+// once.  A thread reads 8 (FP64: 4) consecutive k of one row of A (lanes down
+// the column) and stores them as 16-byte rows; in BF16X3 mode the split into
+// the two terms happens there, once per element instead of once per
+// wavefront that uses it.  Addresses are clamped into the matrices, only the
+// tail of K is zeroed: what a lane past m or n computes is not stored.  The
+// products are formed transposed (lane % 16 = row of C), so C leaves the
+// accumulators in contiguous runs without passing through LDS.
+// Workgroups are numbered so that each XCD (workgroup id % 8) takes a
+// contiguous range of tiles, whose operands its L2 then holds.
+// One wavefront per workgroup (WV = 1) where m and n are at most 32: a 64x64
+// tile would leave three of its four wavefronts without a column.
+// Against one chunk at a time through one buffer and scalar LDS stores: 1500 x
+// 1100 x 1300 in FP64 254 -> 117 us, 2000 split-BF16 products of 100 x 75 x 50
+// 92 -> 51 us, 16384 FP32 products of 12 x 9 x 20 67 -> 18 us, bit for bit.
 template <typename T, int MODE>
-__global__ __launch_bounds__(kThreads) void gemm_tiled_kernel(int m, int n, int k, T alpha,
-                                                              const T *__restrict__ A, int64_t lda,
-                                                              int64_t strideA,
-                                                              const T *__restrict__ B, int64_t ldb,
-                                                              int64_t strideB, T beta, T *C,
-                                                              int64_t ldc, int64_t strideC,
-                                                              int tiles_m, int64_t batch) {
-    constexpr int TK = Cfg<T>::TK, S = Cfg<T>::S;
-    __shared__ __attribute__((aligned(16))) T smem[2 * kTM * S > kTM * (kTN + 1) ? 2 * kTM * S : kTM * (kTN + 1)];
-    T *As = smem, *Bs = smem + kTM * S;
+struct Chunk {
+    static constexpr bool kSplit = MODE == GPUTILS_GEMM_BF16X3;
+    static constexpr int TK = sizeof(T) == 8 ? 16 : 32;  // k per chunk
+    static constexpr int PT = sizeof(T) == 8 ? 4 : 8;    // consecutive k of a thread's row of A
+    // LDS row stride in elements: 16-byte aligned rows, operand reads of 16
+    // rows x 4 k on distinct banks (bf16: two planes)
+    static constexpr int S = TK + (kSplit ? 8 : sizeof(T) == 8 ? 2 : 4);
+    using lds_t = std::conditional_t<kSplit, __bf16, T>;
+    static constexpr int kPlanes = kSplit ? 2 : 1;
+};
+
+template <typename T, int MODE, int WV>
+__global__ __launch_bounds__(64 * WV *WV) __attribute__((amdgpu_waves_per_eu(4))) void gemm_tiled_kernel(int m, int n, int k, T alpha,
+                                                                 const T *__restrict__ A, int64_t lda,
+                                                                 int64_t strideA, const T *__restrict__ B,
+                                                                 int64_t ldb, int64_t strideB, T beta, T *C,
+                                                                 int64_t ldc, int64_t strideC, int tiles_m,
+                                                                 int tiles, int64_t batch) {
+    using Ch = Chunk<T, MODE>;
     using M = Mfma16<T>;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = 32 * (wave & 1), wn = 32 * (wave >> 1);
-    const int i0 = (blockIdx.x % tiles_m) * kTM, j0 = (blockIdx.x / tiles_m) * kTN;
+    using E = typename Ch::lds_t;
+    constexpr int kTile = 32 * WV, kNt = 64 * WV * WV, TK = Ch::TK, PT = Ch::PT, S = Ch::S;
+    constexpr int kPlane = kTile * S;  // elements of one operand plane
+    constexpr int kBufs = WV == 1 ? 1 : 2;  // one wavefront needs no second buffer: its own order is enough
+    __shared__ __attribute__((aligned(16))) E smem[kBufs][2 * Ch::kPlanes * kPlane];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = 32 * (wave % WV), wn = 32 * (wave / WV);
+    int tile = blockIdx.x;
+    if (tiles >= 64) {  // a contiguous range of tiles per XCD, the remainder as it comes
+        const int per = tiles >> 3;
+        if (tile < 8 * per) tile = (tile & 7) * per + (tile >> 3);
+    }
+    const int i0 = (tile % tiles_m) * kTile, j0 = (tile / tiles_m) * kTile;
     const int64_t bidx = blockIdx.y + (int64_t)blockIdx.z * 65535;
     if (bidx >= batch) return;  // uniform per workgroup
-    const T *a = A + bidx * strideA;
-    const T *b = B + bidx * strideB;
     T *c = C + bidx * strideC;
 
-    typename M::acc_t acc[2][2];
+    // A: row tid % kTile, k = PT * (tid / kTile) .. ; B: k = tid % TK, columns
+    // tid / TK + kNt / TK * u
+    constexpr int kAU = kTile * TK / (kNt * PT), kBU = kTile * TK / kNt;
+    const int ar = tid % kTile, ak = PT * (tid / kTile), br = tid % TK, bj = tid / TK;
+    const T *a = A + bidx * strideA + (i0 + ar < m ? i0 + ar : m - 1);
+    const T *b = B + bidx * strideB;
+    T va[kAU][PT], vb[kBU];
+    auto fetch = [&](int k0) {
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+        for (int q = 0; q < kAU; ++q)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = M::zero();
-
-    for (int k0 = 0; k0 < k; k0 += TK) {
-        __syncthreads();
-        stage<T>(a, lda, b, ldb, m, n, k, i0, j0, k0, As, Bs);
-        __syncthreads();
-        if constexpr (MODE == GPUTILS_GEMM_BF16X3) {
-            // one 16x16x32 step per tile: lane holds 8 consecutive k
-            const int r = lane & 15, g = lane >> 4;
-            bf16x8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-                const float4 *pa = reinterpret_cast<const float4 *>(As + (wm + 16 * x + r) * S + 8 * g);
-                const float4 *pb = reinterpret_cast<const float4 *>(Bs + (wn + 16 * x + r) * S + 8 * g);
-                float va[8], vb[8];
-                const float4 a0 = pa[0], a1 = pa[1], b0 = pb[0], b1 = pb[1];
-                va[0] = a0.x; va[1] = a0.y; va[2] = a0.z; va[3] = a0.w;
-                va[4] = a1.x; va[5] = a1.y; va[6] = a1.z; va[7] = a1.w;
-                vb[0] = b0.x; vb[1] = b0.y; vb[2] = b0.z; vb[3] = b0.w;
-                vb[4] = b1.x; vb[5] = b1.y; vb[6] = b1.z; vb[7] = b1.w;
-                split_bf16(va, ah[x], al[x]);
-                split_bf16(vb, bh[x], bl[x]);
+            for (int u = 0; u < PT; ++u) {
+                const int kk = k0 + ak + q * (PT * kNt / kTile) + u;
+                va[q][u] = a[(int64_t)(kk < k ? kk : k - 1) * lda];
             }
+        const int kb = k0 + br < k ? k0 + br : k - 1;
 #pragma unroll
-            for (int x = 0; x < 2; ++x)
+        for (int u = 0; u < kBU; ++u) {
+            const int j = j0 + bj + (kNt / TK) * u;
+            vb[u] = b[kb + (int64_t)(j < n ? j : n - 1) * ldb];
+        }
+        if (k0 + TK > k) {  // uniform: the tail of K is zero in both operands
 #pragma unroll
-                for (int y = 0; y < 2; ++y) {
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[x], bh[y], acc[x][y], 0, 0, 0);
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[x], bl[y], acc[x][y], 0, 0, 0);
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[x], bh[y], acc[x][y], 0, 0, 0);
-                }
-        } else {
-            const int r = lane & 15, g = lane >> 4;
+            for (int q = 0; q < kAU; ++q)
 #pragma unroll
-            for (int kk = 0; kk < TK; kk += 4) {
-                T av[2], bv[2];
+                for (int u = 0; u < PT; ++u)
+                    if (k0 + ak + q * (PT * kNt / kTile) + u >= k) va[q][u] = T(0);
+            if (k0 + br >= k) {
 #pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    av[x] = As[(wm + 16 * x + r) * S + kk + g];
-                    bv[x] = Bs[(wn + 16 * x + r) * S + kk + g];
-                }
-#pragma unroll
-                for (int x = 0; x < 2; ++x)
-#pragma unroll
-                    for (int y = 0; y < 2; ++y) acc[x][y] = M::fma(av[x], bv[y], acc[x][y]);
+                for (int u = 0; u < kBU; ++u) vb[u] = T(0);
             }
         }
-    }
-    // stage the 64x64 tile column-major (ld 65) and write coalesced
-    __syncthreads();
-    T *Cs = smem;
-    {
-        const int col = lane & 15;
+    };
+    auto put = [&](E *buf) {
+        E *As = buf, *Bs = buf + Ch::kPlanes * kPlane;
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
+        for (int q = 0; q < kAU; ++q) {
+            E *row = As + ar * S + ak + q * (PT * kNt / kTile);
+            if constexpr (Ch::kSplit) {
+                bf16x8 hi, lo;
+                split_bf16(va[q], hi, lo);
+                *reinterpret_cast<bf16x8 *>(row) = hi;
+                *reinterpret_cast<bf16x8 *>(row + kPlane) = lo;
+            } else {
+                typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
 #pragma unroll
-            for (int y = 0; y < 2; ++y)
+                for (int u = 0; u < PT; u += 16 / (int)sizeof(T)) {
+                    vec v;
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    Cs[(wm + 16 * x + M::drow(lane, r)) + (wn + 16 * y + col) * (kTM + 1)] = acc[x][y][r];
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < kTM * kTN; e += kThreads) {
-        const int i = e % kTM, j = e / kTM;
-        const int gi = i0 + i, gj = j0 + j;
-        if (gi < m && gj < n) {
-            T v = alpha * Cs[i + j * (kTM + 1)];
-            T *dst = c + gi + (int64_t)gj * ldc;
-            if (beta != T(0)) v += beta * *dst;
-            *dst = v;
+                    for (int e = 0; e < 16 / (int)sizeof(T); ++e) v[e] = va[q][u + e];
+                    *reinterpret_cast<vec *>(row + u) = v;
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kBU; ++u) {
+            E *p = Bs + (bj + (kNt / TK) * u) * S + br;
+            if constexpr (Ch::kSplit) {
+                const __bf16 h = (__bf16)vb[u];
+                *p = h;
+                p[kPlane] = (__bf16)(vb[u] - (float)h);
+            } else {
+                *p = vb[u];
+            }
+        }
+    };
+
+    const int r = lane & 15, g = lane >> 4;
+    // The whole loop for NX x NY of the wavefront's 16x16 tiles inside C:
+    // acc[y][x] holds columns wn + 16 y, rows wm + 16 x of C, transposed.  One
+    // loop per count, so that no branch splits the accumulators; wavefronts
+    // with other counts meet at the same barriers.
+    auto product = [&](auto nx_c, auto ny_c) {
+        constexpr int NX = decltype(nx_c)::value, NY = decltype(ny_c)::value;
+        typename M::acc_t acc[NY > 0 ? NY : 1][NX > 0 ? NX : 1];
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+#pragma unroll
+            for (int x = 0; x < NX; ++x) acc[y][x] = M::zero();
+        auto multiply = [&](const E *buf, int left) {  // left: k from this chunk on
+            const E *As = buf + (wm + r) * S, *Bs = buf + Ch::kPlanes * kPlane + (wn + r) * S;
+            if constexpr (NX == 0 || NY == 0) return;
+            else if constexpr (Ch::kSplit) {
+                // one 16x16x32 step: lane holds 8 consecutive k
+                bf16x8 ah[NX], al[NX], bh[NY], bl[NY];
+#pragma unroll
+                for (int x = 0; x < NX; ++x) {
+                    ah[x] = *reinterpret_cast<const bf16x8 *>(As + 16 * x * S + 8 * g);
+                    al[x] = *reinterpret_cast<const bf16x8 *>(As + 16 * x * S + 8 * g + kPlane);
+                }
+#pragma unroll
+                for (int y = 0; y < NY; ++y) {
+                    bh[y] = *reinterpret_cast<const bf16x8 *>(Bs + 16 * y * S + 8 * g);
+                    bl[y] = *reinterpret_cast<const bf16x8 *>(Bs + 16 * y * S + 8 * g + kPlane);
+                }
+#pragma unroll
+                for (int y = 0; y < NY; ++y)
+#pragma unroll
+                    for (int x = 0; x < NX; ++x) {
+                        acc[y][x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[y], al[x], acc[y][x], 0, 0, 0);
+                        acc[y][x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[y], ah[x], acc[y][x], 0, 0, 0);
+                        acc[y][x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[y], ah[x], acc[y][x], 0, 0, 0);
+                    }
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < TK; kk += 4) {
+                    if (kk > 0 && kk >= left) break;  // uniform; left is known to reach TK inside the loop
+                    T av[NX], bv[NY];
+#pragma unroll
+                    for (int x = 0; x < NX; ++x) av[x] = As[16 * x * S + kk + g];
+#pragma unroll
+                    for (int y = 0; y < NY; ++y) bv[y] = Bs[16 * y * S + kk + g];
+#pragma unroll
+                    for (int y = 0; y < NY; ++y)
+#pragma unroll
+                        for (int x = 0; x < NX; ++x) acc[y][x] = M::fma(bv[y], av[x], acc[y][x]);
+                }
+            }
+        };
+        fetch(0);  // k >= 1 (the caller)
+        put(smem[0]);
+        __syncthreads();
+        int cur = 0, k0 = 0;
+        for (; k0 + TK < k; k0 += TK, cur ^= kBufs - 1) {
+            fetch(k0 + TK);
+            multiply(smem[cur], TK);
+            if constexpr (kBufs == 1) __syncthreads();
+            put(smem[cur ^ (kBufs - 1)]);
+            __syncthreads();
+        }
+        multiply(smem[cur], k - k0);
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+#pragma unroll
+            for (int x = 0; x < NX; ++x) {
+                const int gi = i0 + wm + 16 * x + r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int gj = j0 + wn + 16 * y + M::drow(lane, e);
+                    if (gi < m && gj < n) {
+                        T *dst = c + gi + (int64_t)gj * ldc;
+                        T v = alpha * acc[y][x][e];
+                        if (beta != T(0)) v += beta * *dst;
+                        *dst = v;
+                    }
+                }
+            }
+    };
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    const int mr = m - (i0 + wm), nr = n - (j0 + wn);
+    if (mr > 16 && nr > 16) product(Two(), Two());
+    else if (mr <= 0 || nr <= 0) product(Zero(), Zero());
+    else if (nr > 16) product(One(), Two());
+    else if (mr > 16) product(Two(), One());
+    else product(One(), One());
+}
+
+// C <- beta C (k = 0: the product is empty).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void gemm_scale_kernel(int m, int n, T beta, T *C, int64_t ldc,
+                                                              int64_t strideC, int64_t batch) {
+    const int64_t total = (int64_t)m * n;
+    for (int64_t b = blockIdx.x; b < batch; b += gridDim.x) {
+        T *c = C + b * strideC;
+        for (int64_t e = threadIdx.x; e < total; e += kThreads) {
+            T *dst = c + e % m + (e / m) * ldc;
+            *dst = (beta != T(0)) ? beta * *dst : T(0);
         }
     }
 }
@@ -593,7 +690,14 @@ int run(int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, int64
             return launch_check("gemm_reg_kernel");
         }
     }
-    const int tiles_m = (int)ceil_div(m, kTM), tiles_n = (int)ceil_div(n, kTN);
+    if (k == 0) {
+        hipLaunchKernelGGL((gemm_scale_kernel<T>), dim3(grid_1d(batch, 1)), dim3(kThreads), 0, st, (int)m, (int)n,
+                           beta, C, ldc, strideC, batch);
+        return launch_check("gemm_scale_kernel");
+    }
+    const bool small = m <= 32 && n <= 32;
+    const int tile = small ? 32 : 64;
+    const int tiles_m = (int)ceil_div(m, tile), tiles_n = (int)ceil_div(n, tile);
     const int64_t tiles = (int64_t)tiles_m * tiles_n;
     if (tiles > 0x7fffffff) {
         set_error("gemm: too many tiles");
@@ -601,9 +705,9 @@ int run(int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, int64
     }
     const unsigned gy = (unsigned)(batch < 65535 ? batch : 65535);
     const unsigned gz = (unsigned)ceil_div(batch, 65535);
-    hipLaunchKernelGGL((gemm_tiled_kernel<T, MODE>), dim3((unsigned)tiles, gy, gz), dim3(kThreads), 0,
-                       st, (int)m, (int)n, (int)k, alpha, A, lda, strideA, B, ldb, strideB, beta, C,
-                       ldc, strideC, tiles_m, batch);
+    hipLaunchKernelGGL((small ? gemm_tiled_kernel<T, MODE, 1> : gemm_tiled_kernel<T, MODE, 2>),
+                       dim3((unsigned)tiles, gy, gz), dim3(small ? 64 : 256), 0, st, (int)m, (int)n, (int)k, alpha, A,
+                       lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, tiles_m, (int)tiles, batch);
     return launch_check("gemm_tiled_kernel");
 }
 
