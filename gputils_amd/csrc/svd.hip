@@ -46,6 +46,7 @@
 
 #include "common.hpp"
 #include "householder.hpp"
+#include "qr_regs.hpp"
 
 namespace gputils {
 namespace svd {
@@ -583,6 +584,27 @@ __device__ int fp32_first_sweeps(double *W, double *X, int n, bool lower, double
     return s32;
 }
 
+// FP64 QR of the m x n matrix a with its columns in registers (RegQr, 16
+// lanes a column), the factors to G (ld m) and tau.  Streaming the trailing
+// columns through LDS for every reflector took 162 us of a 96 x 48 matrix's
+// 808 (four workgroups per CU, issue-bound): @SVDQR@.
+template <int KR, int SL, typename T>
+__device__ __forceinline__ void factor_columns(const T *__restrict__ a, int64_t lda, int m, int n, double *G,
+                                               double *vbuf, double *s_tau, double *tau) {
+    using Q = qrr::RegQr<double, double, double, 16, kThreads / kWave, KR, SL>;
+    Q qr;
+#pragma unroll
+    for (int q = 0; q < SL; ++q) {
+        const int c = qr.col(q);
+        qr.load(q, a + (int64_t)(c < n ? c : 0) * lda, m, c < n);
+        asm volatile("" ::: "memory");  // one slot's loads in flight at a time
+    }
+    qr.factor(n, n, vbuf, s_tau, tau);
+#pragma unroll
+    for (int q = 0; q < SL; ++q) qr.store(q, G + (int64_t)qr.col(q) * m, m, qr.col(q) < n);
+    __syncthreads();
+}
+
 template <typename T, int MODE, bool MIXED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void gesvd_kernel(int m, int n, const T *__restrict__ A, int64_t lda,
                                                          int64_t strideA, T *S, int64_t strideS, T *U,
@@ -608,13 +630,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 
     // 1. stage and factorise
     const T *a = A + b * strideA;
-    for (int e = tid; e < m * n; e += kThreads) {
-        const int i = e % m, j = e / m;
-        G[i + (int64_t)j * m] = (double)a[i + (int64_t)j * lda];
+    // the reflector buffers (32 KR doubles) lie in W's and V's space, which
+    // G may share: it is written only after the last barrier
+    double *vbuf = MODE == kWide ? nullptr : lds + L.w;
+    const int64_t free_lds = L.ws + (int64_t)n * n;
+    if (MODE != kWide && m <= 64 && n <= 32 && free_lds >= 32 * 4) {
+        factor_columns<4, 2>(a, lda, m, n, G, vbuf, s_tau, tau);
+    } else if (MODE != kWide && m <= 96 && free_lds >= 32 * 6) {
+        // (taller ones would need more registers than four wavefronts per
+        // SIMD have: 8 row groups x 4 slots spilled 150 of them and made
+        // 80 x 50 slower than through LDS, 831 -> 1025 us for 512)
+        factor_columns<6, 4>(a, lda, m, n, G, vbuf, s_tau, tau);
+    } else {
+        for (int e = tid; e < m * n; e += kThreads) {
+            const int i = e % m, j = e / m;
+            G[i + (int64_t)j * m] = (double)a[i + (int64_t)j * lda];
+        }
+        __syncthreads();
+        if (m <= 16 * 8 + 1) hh::hqr_factor<double, double, double, hh::kWaves, 8>(G, m, m, n, tau, s_tau);
+        else hh::hqr_factor<double, double>(G, m, m, n, tau, s_tau);
     }
-    __syncthreads();
-    if (m <= 16 * 8 + 1) hh::hqr_factor<double, double, double, hh::kWaves, 8>(G, m, m, n, tau, s_tau);
-    else hh::hqr_factor<double, double>(G, m, m, n, tau, s_tau);
     // VT == NULL (no right singular vectors): the sweeps run on W = R^T, so
     // that the accumulated rotations X are the left singular vectors of R
     // (R^T Z = V_R Sigma  =>  R = Z Sigma V_R^T): no completion is needed for
