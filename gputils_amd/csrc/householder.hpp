@@ -148,16 +148,18 @@ __device__ __forceinline__ void apply_reflector_col(T *A, int64_t lda, int m, in
     if (lane == 0) x[j] -= tw;
 }
 
-// x + (x of the lane that DPP control CTRL selects), within 16-lane rows
+// x + (x of the lane that DPP control CTRL selects), within 16-lane rows.
+// mov_dpp leaves no previous value to keep (every lane has a source here), so
+// FP64 takes two moves and an addition, not four moves.
 template <int CTRL>
 __device__ __forceinline__ float row16_plus(float x) {
-    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
 }
 template <int CTRL>
 __device__ __forceinline__ double row16_plus(double x) {
     const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
     return x + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 

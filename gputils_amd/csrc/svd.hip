@@ -165,36 +165,17 @@ __device__ __forceinline__ void jacobi_angle(float al, float be, float ga, float
     sn = cs * t;
 }
 
-// x + (x of the lane that DPP control CTRL selects), within 16-lane rows
-template <int CTRL>
-__device__ __forceinline__ double dpp_plus(double x) {
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
-    return x + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // Sums over aligned groups of 8 / 16 lanes, result in every lane of the
 // group: quad permutations [1,0,3,2] and [2,3,0,1] sum each quad, the row
 // half mirror (lane i <-> 7 - i) adds the other quad of the 8, the row
 // mirror (lane i <-> 15 - i) the other 8 of the 16.  Register moves only.
-__device__ __forceinline__ double group8_sum(double x) {
-    x = dpp_plus<0xB1>(x);      // quad_perm [1,0,3,2]
-    x = dpp_plus<0x4E>(x);      // quad_perm [2,3,0,1]
-    return dpp_plus<0x141>(x);  // row_half_mirror
+template <typename R>
+__device__ __forceinline__ R group8_sum(R x) {
+    x = hh::row16_plus<0xB1>(x);      // quad_perm [1,0,3,2]
+    x = hh::row16_plus<0x4E>(x);      // quad_perm [2,3,0,1]
+    return hh::row16_plus<0x141>(x);  // row_half_mirror
 }
-__device__ __forceinline__ double group16_sum(double x) {
-    return dpp_plus<0x140>(group8_sum(x));  // row_mirror
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_plus(float x) {
-    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float group8_sum(float x) {
-    x = dpp_plus<0xB1>(x);
-    x = dpp_plus<0x4E>(x);
-    return dpp_plus<0x141>(x);
-}
+__device__ __forceinline__ double group16_sum(double x) { return hh::row16_sum(x); }
 
 // Pair i of round r in a round-robin tournament over n2 (even) players:
 // player 0 is fixed, players 1..n2-1 rotate.  Every unordered pair meets
@@ -476,10 +457,20 @@ __device__ __forceinline__ bool jacobi_sweeps_k(R *W, R *X, int n, R tol2, R sto
     return converged;
 }
 
-template <typename R, int MODE>
+template <typename R, int MODE, bool COARSE>
 __device__ __forceinline__ bool jacobi_sweeps(R *W, R *X, int n, R tol2, R stop2, int max_sweeps, int &sweeps,
                                               double *gdiag = nullptr) {
     if constexpr (MODE != kWide) {
+        // as many entries per lane as the columns need: each is loaded,
+        // multiplied and stored in every round (512 FP64 80 x 50 decompositions
+        // with 8 entries 786 us, with 7 746).  The mixed kernels, which
+        // hold the FP32 and the FP64 sweeps, take every second count only:
+        // with all of them their registers went to scratch.
+        if constexpr (!COARSE) {
+            if (n <= 16) return jacobi_sweeps_k<R, MODE, 2>(W, X, n, tol2, stop2, max_sweeps, sweeps, gdiag);
+            if (n > 32 && n <= 40) return jacobi_sweeps_k<R, MODE, 5>(W, X, n, tol2, stop2, max_sweeps, sweeps, gdiag);
+            if (n > 48 && n <= 56) return jacobi_sweeps_k<R, MODE, 7>(W, X, n, tol2, stop2, max_sweeps, sweeps, gdiag);
+        }
         if (n <= 32) return jacobi_sweeps_k<R, MODE, 4>(W, X, n, tol2, stop2, max_sweeps, sweeps, gdiag);
         if (n <= 48) return jacobi_sweeps_k<R, MODE, 6>(W, X, n, tol2, stop2, max_sweeps, sweeps, gdiag);
     }
@@ -529,7 +520,7 @@ __device__ int fp32_first_sweeps(double *W, double *X, int n, bool lower, double
         // take it from there in as many sweeps as from the FP32-converged
         // state (the last FP32 sweeps before convergence are saved)
         const float tol = (float)(n > 2 ? n : 2) * FLT_EPSILON;
-        jacobi_sweeps<float, MODE>(W32, X32, n, tol * tol, 1e-4f, kMaxSweeps, s32);
+        jacobi_sweeps<float, MODE, true>(W32, X32, n, tol * tol, 1e-4f, kMaxSweeps, s32);
         float *F = W32;  // W32 is not needed any more
         for (int e = tid; e < nn; e += kThreads) {
             const int i = e % n, j = e / n;
@@ -587,7 +578,7 @@ __device__ int fp32_first_sweeps(double *W, double *X, int n, bool lower, double
 // FP64 QR of the m x n matrix a with its columns in registers (RegQr, 16
 // lanes a column), the factors to G (ld m) and tau.  Streaming the trailing
 // columns through LDS for every reflector took 162 us of a 96 x 48 matrix's
-// 808 (four workgroups per CU, issue-bound): @SVDQR@.
+// 808 (four workgroups per CU, issue-bound); 2048 null spaces 1730 -> 1632 us.
 template <int KR, int SL, typename T>
 __device__ __forceinline__ void factor_columns(const T *__restrict__ a, int64_t lda, int m, int n, double *G,
                                                double *vbuf, double *s_tau, double *tau) {
@@ -701,7 +692,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const double tol = (double)(n > 2 ? n : 2) * DBL_EPSILON;
     // sig (n doubles, free until the singular values) carries the Gram
     // diagonal of the convergence test
-    const bool converged = jacobi_sweeps<double, MODE>(W, X, n, tol * tol, tol * tol, kMaxSweeps, s64, sig);
+    const bool converged = jacobi_sweeps<double, MODE, MIXED>(W, X, n, tol * tol, tol * tol, kMaxSweeps, s64, sig);
     __syncthreads();
 
     // 3. singular values, order, signs
