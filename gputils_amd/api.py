@@ -36,11 +36,13 @@ def to_matrices(t: torch.Tensor) -> torch.Tensor:
 
 
 def stream_handle() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle itself: torch.cuda.current_stream() builds a Stream object around it
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    # every pointer argument is declared c_void_p, which takes the integer
+    return t.data_ptr() if t is not None else None
 
 
 def _check_dev(t: torch.Tensor, name: str, dtypes=(torch.float32, torch.float64)):
@@ -127,7 +129,9 @@ def gemm_batched(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor | None = None
     batch, kk, m = A.shape
     n = B.shape[1]
     if C is None:
-        C = torch.zeros((batch, n, m), dtype=A.dtype, device=A.device)
+        # with beta = 0 every kernel writes all of C and reads none of it; filling it
+        # took 10 of 62 us for 2000 products of 100x50 by 50x75 in FP32
+        C = (torch.empty if beta == 0 else torch.zeros)((batch, n, m), dtype=A.dtype, device=A.device)
     _check_dev(C, "C")
     st = stream_handle()
     if A.dtype == torch.float64:
@@ -145,10 +149,9 @@ _WS = {}
 
 
 def _workspace(device) -> torch.Tensor:
-    key = str(device)
-    if key not in _WS:
-        _WS[key] = torch.empty(lib().gputils_reduce_workspace_bytes(), dtype=torch.uint8, device=device)
-    return _WS[key]
+    if device not in _WS:
+        _WS[device] = torch.empty(lib().gputils_reduce_workspace_bytes(), dtype=torch.uint8, device=device)
+    return _WS[device]
 
 
 def _reduce(name, x, y=None):

@@ -51,3 +51,16 @@ def test_padded_products(m, n, k, mode, alpha, beta):
     tol = (k + 2) * u + (2.0 ** -15 if mode == "bf16x3" else 0.0)
     assert np.all(np.abs(got[:, :, :m] - ref) <= tol * size + 1e-300)
     assert np.isnan(got[:, :, m:]).all()
+
+
+# one shape per route: whole matrices in LDS, registers, a vector, small odd shapes, tiles
+@pytest.mark.parametrize("m,n,k", [(64, 64, 64), (128, 128, 128), (64, 1, 64), (5, 3, 7), (100, 50, 75), (200, 17, 129)])
+@pytest.mark.parametrize("dtype,mode", [(torch.float32, "fp32"), (torch.float32, "bf16x3"), (torch.float64, "fp32")])
+def test_new_result_is_written_whole(m, n, k, dtype, mode):
+    r = np.random.default_rng(m * n + k)
+    A = torch.from_numpy(r.standard_normal((3, k, m))).to(dtype).cuda()
+    B = torch.from_numpy(r.standard_normal((3, n, k))).to(dtype).cuda()
+    want = api.gemm_batched(A, B, torch.zeros(3, n, m, dtype=dtype, device="cuda"), mode=mode)
+    old = torch.full((3, n, m), float("nan"), dtype=dtype, device="cuda")
+    del old  # the allocator hands this block to the next result of its size
+    assert torch.equal(api.gemm_batched(A, B, mode=mode), want)
