@@ -456,7 +456,7 @@ __device__ __forceinline__ void ragged_factor(const double *__restrict__ a, cons
     if constexpr (64 * LPC * KR > kMin) {
         constexpr int kMaxCols = (MAXE / (MLO + 1) < 64 ? MAXE / (MLO + 1) : 64) + 1;
         constexpr int kStep = NW * (kWave / LPC);
-        using Q = qrr::RegQr<float, double, float, LPC, NW, KR, (kMaxCols + kStep - 1) / kStep>;
+        using Q = qrr::RegQr<float, double, float, LPC, NW, KR, (kMaxCols + kStep - 1) / kStep, 64>;
         static_assert(Q::kV <= 1024, "the reflectors share rd's LDS");
         Q qr;
 #pragma unroll
@@ -471,6 +471,17 @@ __device__ __forceinline__ void ragged_factor(const double *__restrict__ a, cons
         for (int q = 0; q < Q::kSlots; ++q)
             if (qr.first(q) <= n) qr.store(q, S + qr.col(q) * m, m, qr.col(q) <= n);
     }
+}
+
+// Wavefronts per SIMD to leave registers for: in the smaller buckets one
+// register too many (129 where 128 fit) costs a workgroup per CU, 1089 against
+// 1065 us for 4096 systems of 8 to 64 columns.
+constexpr int ragged_waves(int maxe, int nw, int method) {
+    const int least = nw < 4 ? 1 : nw / 4;
+    if (method != 0) return least;
+    const int fit = maxe == 2048 ? (nw == 2 ? 3 : 4) : maxe == 4096 ? (nw >= 8 ? 4 : nw == 4 ? 3 : 2)
+                  : maxe == 8192 ? (nw == 8 ? 3 : nw == 4 ? 2 : 1) : 1;
+    return fit > least ? fit : least;
 }
 
 // One bucket of the ragged plan: workgroup w solves the items
@@ -493,13 +504,13 @@ __device__ __forceinline__ void ragged_factor(const double *__restrict__ a, cons
 // 0 is bound by the chain of the reflector (about 1350 cycles for short
 // columns) and for tall ones by issue; with A streamed from LDS for every
 // column it took 3700 to 5300.  4096 systems of the configuration, one
-// refinement step: default shapes 1547 -> 1035 us, tuned 1112 -> 809 us.  The plan
+// refinement step: default shapes 1533 -> 1071 us, tuned 1119 -> 855 us.  The plan
 // picks METHOD, NW and the grid per bucket.  For one METHOD every system's
 // arithmetic is the same for every NW and every item-to-workgroup
 // assignment, so the results are too; the two methods round the FP32
 // factorisation differently.
 template <int MAXE, int NW, int METHOD>
-__global__ __launch_bounds__(NW * kWave) void gels_ragged_kernel(const RaggedItem *__restrict__ items,
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(ragged_waves(MAXE, NW, METHOD)))) void gels_ragged_kernel(const RaggedItem *__restrict__ items,
                                                                const int *__restrict__ wstart,
                                                                const double *__restrict__ A, double *B,
                                                                int steps, int *queue) {

@@ -108,9 +108,9 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
 
 // C <- Q^T C (trans) or Q C, Q from k reflectors.  A wavefront holds SL
 // columns of C in registers (rows lane + 64 u, u < R) for all the
-// reflectors; the workgroup stages kChunk of them at a time in LDS, as whole
-// vectors [0 .. 0, 1, v], the next ones already on their way.  Bound by the
-// chain of a reflector (its LDS reads, one wave reduction, the update), so
+// reflectors; the workgroup stages kChunk of them at a time in LDS, as
+// vectors [0 .. 0, 0, v] without the unit entry, the next ones already on
+// their way.  Bound by the chain of a reflector (its LDS reads, one wave reduction, the update), so
 // few columns go one to a wavefront over as many workgroups as there are;
 // batches that fill the chip take four.  tau NULL: the scalar is formed from
 // the vector, tau = 2 / (1 + |v|^2), or 0 for v = 0 (H = I): least squares has
@@ -147,16 +147,39 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
         for (int u = 0; u < R; ++u)
             if (lane + kWave * u >= m) x[s][u] = T(0);
     }
-    // chunk q of reflectors in the order they are applied: entry e of the
-    // chunk is reflector refl(q, e); wavefront w stages entries w and w + 4
-    auto refl = [&](int q, int e) { return trans ? q * kChunk + e : k - 1 - (q * kChunk + e); };
+    // chunk q of reflectors in the order they are applied (aligned to kChunk):
+    // entry e of its ne(q) is reflector refl(q, e); wavefront w stages entries
+    // w and w + 4
+    const int chunks = (k + kChunk - 1) / kChunk;
+    auto base = [&](int q) { return (trans ? q : chunks - 1 - q) * kChunk; };
+    auto count = [&](int q) { return k - base(q) < kChunk ? k - base(q) : kChunk; };
+    auto refl = [&](int q, int e) { return trans ? base(q) + e : base(q) + count(q) - 1 - e; };
+    // The rows of a chunk's unit entries lie in one block of 64: it and block 0
+    // change places in the registers and in V, so that the unit entry is always
+    // in slot 0.  Its product joins the dot product after the reduction (see
+    // RegQr).  A 600 x 150 FP64 QR, solution and Q take 405 us so, as with the
+    // entry in the lanes' sums, and 458 with the row's register selected in
+    // every step.
+    int head = 0;  // block in slot 0
+    auto swap0 = [&](int u0) {
+#pragma unroll
+        for (int u = 1; u < R; ++u) {
+            const bool take = u == u0;  // uniform; selects, as a branch would index x (scratch)
+#pragma unroll
+            for (int s = 0; s < SL; ++s) {
+                const T y = x[s][0], z = x[s][u];
+                x[s][0] = take ? z : y;
+                x[s][u] = take ? y : z;
+            }
+        }
+    };
     constexpr int kPer = kChunk / kOrmWaves;
     T nv[kPer][R];
     auto fetch = [&](int q) {
 #pragma unroll
         for (int p = 0; p < kPer; ++p) {
             const int e = wave + kOrmWaves * p;
-            const int j = q * kChunk + e < k ? refl(q, e) : 0;
+            const int j = e < count(q) ? refl(q, e) : 0;
             const T *col = a + (int64_t)j * lda;
 #pragma unroll
             for (int u = 0; u < R; ++u) {
@@ -165,11 +188,10 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
             }
         }
     };
-    const int chunks = (k + kChunk - 1) / kChunk;
     fetch(0);
 #pragma unroll 1
     for (int q = 0; q < chunks; ++q) {
-        const int ne = k - q * kChunk < kChunk ? k - q * kChunk : kChunk;
+        const int ne = count(q), ju = base(q) / kWave;
 #pragma unroll
         for (int p = 0; p < kPer; ++p) {
             const int e = wave + kOrmWaves * p;
@@ -180,7 +202,7 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
                 const int i = lane + kWave * u;
                 const T v = (i > j && i < m) ? nv[p][u] : T(0);
                 vv = fma(v, v, vv);
-                V[e][i] = (i == j) ? T(1) : v;
+                V[e][lane + kWave * (u == ju ? 0 : u == 0 ? ju : u)] = v;
             }
             if (tau == nullptr) {  // uniform
                 vv = wave_sum(vv);
@@ -190,14 +212,22 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
         if (tau != nullptr && (int)threadIdx.x < ne) s_tau[threadIdx.x] = tb[refl(q, threadIdx.x)];
         __syncthreads();
         if (q + 1 < chunks) fetch(q + 1);
+        if (ju != head) {  // uniform
+            swap0(head);
+            swap0(ju);
+            head = ju;
+        }
         if (c0 < ncols) {  // uniform
 #pragma unroll 1
             for (int e = 0; e < ne; ++e) {
+                const int jl = refl(q, e) & (kWave - 1);
                 T vr[R];
 #pragma unroll
                 for (int u = 0; u < R; ++u) vr[u] = V[e][lane + kWave * u];
                 const T t = s_tau[e];
-                T w[SL];
+                T w[SL], xj[SL];
+#pragma unroll
+                for (int s = 0; s < SL; ++s) xj[s] = readlane(x[s][0], jl);
 #pragma unroll
                 for (int s = 0; s < SL; ++s) {
                     T w0 = T(0), w1 = T(0);
@@ -208,8 +238,9 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
                     }
                     w[s] = w0 + w1;
                 }
+                if (lane == jl) vr[0] = T(1);
 #pragma unroll
-                for (int s = 0; s < SL; ++s) w[s] = t * wave_sum(w[s]);
+                for (int s = 0; s < SL; ++s) w[s] = t * (wave_sum(w[s]) + xj[s]);
                 if (t != T(0)) {  // H = I stays out of C
 #pragma unroll
                     for (int s = 0; s < SL; ++s)
@@ -220,6 +251,7 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
         }
         __syncthreads();
     }
+    swap0(head);
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
         if (c0 + s >= ncols) continue;

@@ -85,12 +85,18 @@ __device__ __forceinline__ void scalars(double alpha, double sq, double &beta, d
 // wavefronts.  LPC = 16 makes a reduction four steps for four columns; 64
 // takes less registers for the reflector that everybody holds, and is for
 // the taller matrices.
-template <typename T, typename ACC, typename DOT, int LPC, int NW, int KR, int SL>
+// NMAX bounds the reflectors, n.  The unit entry of a reflector stays out of the
+// lanes' chains, and its product joins the dot product after the reduction:
+// it is the largest term, and partial sums that hold it round at its size
+// (error against 64 bits of 2500 FP32 systems of 65 to 128 rows 6 % larger).
+// NMAX = 0 leaves it in them, for a caller whose errors are set elsewhere.
+template <typename T, typename ACC, typename DOT, int LPC, int NW, int KR, int SL, int NMAX = NW * (kWave / LPC) * SL>
 struct RegQr {
     static constexpr int kGroups = kWave / LPC;      // columns of one slot of a wavefront
     static constexpr int kCols = NW * kGroups * SL;  // columns held
     static constexpr int kSlots = SL;
     static constexpr int kRows = LPC * KR;
+    static constexpr int kUnit = (NMAX + LPC - 1) / LPC < KR ? (NMAX + LPC - 1) / LPC : KR;  // k of row j < kUnit
     static constexpr int kV = 2 * kRows;  // LDS elements of the reflector buffers
     T x[SL][KR];
     int lane, wave, g, l;
@@ -129,8 +135,8 @@ struct RegQr {
     }
 
     // Reflector of column c (this wavefront's slot q): the column becomes
-    // [R; beta; v], vb the whole vector [0 .. 0, 1, v], *s_tau and tau[c] its
-    // scalar.
+    // [R; beta; v], vb the vector [0 .. 0, 0, v] without its unit entry (with
+    // it for kUnit = 0), *s_tau and tau[c] its scalar.
     __device__ __forceinline__ void reflect(T (&xc)[KR], int c, T *vb, T *s_tau, T *tau) {
         const int go = (c / NW) % kGroups;
         T asel = xc[0];
@@ -160,7 +166,7 @@ struct RegQr {
             for (int k = 0; k < KR; ++k) {
                 const int i = l + LPC * k;
                 const T v = xc[k] * scale;
-                vb[i] = (i > c) ? v : ((i == c) ? T(1) : T(0));
+                vb[i] = (i > c) ? v : ((kUnit == 0 && i == c) ? T(1) : T(0));
                 xc[k] = (i > c) ? v : ((i == c) ? (T)beta : xc[k]);
             }
             if (l == 0) {
@@ -170,12 +176,30 @@ struct RegQr {
         }
     }
 
+    // row j of this lane's column
+    __device__ __forceinline__ T row_of(const T (&xc)[KR], int j) const {
+        if constexpr (kUnit == 0) return T(0);
+        T xs = xc[0];
+#pragma unroll
+        for (int k = 1; k < kUnit; ++k)
+            if (k == j / LPC) xs = xc[k];  // uniform
+        if constexpr (LPC == 64) return readlane(xs, j & 63);
+        else return __shfl(xs, (lane & 48) | (j & 15), kWave);
+    }
+    // entry k of the whole reflector of column j
+    __device__ __forceinline__ T whole(const T (&vr)[KR], int k, int j) const {
+        return (k < kUnit && l + LPC * k == j) ? T(1) : vr[k];
+    }
+
     // x_q -= (t v . x_q) v for the columns right of column j in slots Q0 ..
     // Q1 - 1 but slot `skip` (uniform; SL for none): the slots' dot products,
     // their reductions and their updates run side by side
     template <int Q0, int Q1>
     __device__ __forceinline__ void update(int skip, int j, int ntot, const T (&vr)[KR], T t) {
         DOT w[Q1 - Q0];
+        T xj[Q1 - Q0];
+#pragma unroll
+        for (int q = Q0; q < Q1; ++q) xj[q - Q0] = row_of(x[q], j);
 #pragma unroll
         for (int q = Q0; q < Q1; ++q) {
             DOT w0 = DOT(0), w1 = DOT(0);
@@ -188,13 +212,14 @@ struct RegQr {
         }
         if constexpr (LPC == 64) wave_sums(w);
 #pragma unroll
-        for (int q = Q0; q < Q1; ++q) w[q - Q0] = (DOT)t * (LPC == 64 ? w[q - Q0] : hh::row16_sum(w[q - Q0]));
+        for (int q = Q0; q < Q1; ++q)
+            w[q - Q0] = (DOT)t * ((LPC == 64 ? w[q - Q0] : hh::row16_sum(w[q - Q0])) + (DOT)xj[q - Q0]);
 #pragma unroll
         for (int q = Q0; q < Q1; ++q) {
             const int c = col(q);
             if (c > j && c < ntot && q != skip) {
 #pragma unroll
-                for (int k = 0; k < KR; ++k) x[q][k] = fma(-(T)w[q - Q0], vr[k], x[q][k]);
+                for (int k = 0; k < KR; ++k) x[q][k] = fma(-(T)w[q - Q0], whole(vr, k, j), x[q][k]);
             }
         }
     }
@@ -215,6 +240,7 @@ struct RegQr {
     }
     // one slot (the owner's next column)
     __device__ __forceinline__ void update_one(T (&xc)[KR], int c, int j, const T (&vr)[KR], T t) {
+        const T xj = row_of(xc, j);
         DOT w0 = DOT(0), w1 = DOT(0);
 #pragma unroll
         for (int k = 0; k < KR; k += 2) {
@@ -224,10 +250,10 @@ struct RegQr {
         DOT w[1] = {w0 + w1};
         if constexpr (LPC == 64) wave_sums(w);
         else w[0] = hh::row16_sum(w[0]);
-        const T tw = (T)((DOT)t * w[0]);
+        const T tw = (T)((DOT)t * (w[0] + (DOT)xj));
         if (c > j) {
 #pragma unroll
-            for (int k = 0; k < KR; ++k) xc[k] = fma(-tw, vr[k], xc[k]);
+            for (int k = 0; k < KR; ++k) xc[k] = fma(-tw, whole(vr, k, j), xc[k]);
         }
     }
 

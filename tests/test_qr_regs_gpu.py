@@ -113,3 +113,22 @@ def test_more_right_hand_sides_than_one_launch_holds():
     for i in range(k):
         ref = np.linalg.lstsq(A[i], B[i], rcond=None)[0]
         assert np.max(np.abs(X[i] - ref)) <= 1e-11 * np.abs(ref).max()
+
+
+# Column 0 is (0, 1, .., 1): tau = 1 and v_i = 1 / sqrt(m - 1).  The last column
+# is (1, e, .., e) with v_i e = 0.9 half ulps of 1, so R(0, n - 1) = -sqrt(m - 1) e
+# exactly, formed as 1 - (1 + sum).  With the unit entry's product added last the
+# sum rounds twice at size 1 (it, and the scaling by tau); terms summed onto the
+# 1 one by one would all be lost.  Short and tall columns, and a panel's trailing one.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("m,n", [(64, 2), (112, 8), (250, 8), (256, 40), (600, 40), (1024, 40)])
+def test_unit_entry_joins_last(m, n, dtype):
+    u = torch.finfo(dtype).eps / 2
+    A = np.random.default_rng(m + n).standard_normal((m, n))
+    e = float(torch.tensor(0.9 * u * np.sqrt(m - 1)).to(dtype))
+    A[:, 0], A[:, n - 1] = 1.0, e
+    A[0, 0], A[0, n - 1] = 0.0, 1.0
+    tA = torch.from_numpy(np.ascontiguousarray(A.T)[None]).to(dtype).cuda()
+    api.geqrf_batched(tA)
+    got, want = float(tA[0, n - 1, 0]), np.sqrt(m - 1) * e
+    assert abs(abs(got) - want) <= 2.05 * u + 4 * m * u * want
