@@ -85,7 +85,7 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
         const T *src = (c >= n && c < n + nrhs) ? bb + (int64_t)(c - n) * ldb : a + (int64_t)(c < n ? c : 0) * lda;
         qr.load(q, src, m, c < n + nrhs);
     }
-    qr.factor(n, n + nrhs, vbuf, s_tau, taus);
+    qr.factor(n, n + nrhs, vbuf, s_tau, taus, tau == nullptr && nrhs == 0);  // uniform
 #pragma unroll
     for (int q = 0; q < SL; ++q) qr.store(q, a + (int64_t)qr.col(q) * lda, m, qr.col(q) < n);
     if (tau != nullptr)
@@ -113,8 +113,9 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
 // their way.  Bound by the chain of a reflector (its LDS reads, one wave reduction, the update), so
 // few columns go one to a wavefront over as many workgroups as there are;
 // batches that fill the chip take four.  tau NULL: the scalar is formed from
-// the vector, tau = 2 / (1 + |v|^2), or 0 for v = 0 (H = I): least squares has
-// no room to keep it between launches.  Only the first mout rows of C are
+// the vector, tau = 2 / (1 + |v|^2), or 0 for |v|^2 = 0 (H = I): least squares has
+// no room to keep it between launches, and RegQr::reflect sees to it that no
+// other reflector has |v|^2 = 0.  Only the first mout rows of C are
 // written (least squares leaves the rest of b as it was).
 constexpr int kOrmThreads = 256;
 constexpr int kOrmWaves = kOrmThreads / kWave;
