@@ -61,6 +61,26 @@ __device__ __forceinline__ void trsv_regs(const T *R, int ldr, int n, T *c) {
     }
 }
 
+// For reflectors whose scalars will be formed again from v (ormqr_regs_kernel),
+// where |v|^2 = 0 stands for H = I.  A tail so small beside alpha that its square
+// underflows has tau = 2 and beta = -alpha all the same: the first entry of such a
+// v becomes kMark, whose square is a normal number and whose effect lies far below
+// the type's rounding.  Reads back what the workgroup has just stored, and that of
+// reflectors with tau = 2 only, so that it costs the others nothing.
+template <typename T, int NW>
+__device__ __forceinline__ void mark_tails(T *A, int64_t lda, int m, int n, const T *tau) {
+    constexpr T kMark = sizeof(T) == 8 ? T(0x1p-450) : T(0x1p-60);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __syncthreads();
+    for (int c = wave; c < n; c += NW) {
+        if (!(tau[c] > T(1.999))) continue;
+        T *v = A + (int64_t)c * lda;
+        T s = T(0);
+        for (int i = c + 1 + lane; i < m; i += kWave) s = fma(v[i], v[i], s);
+        if (wave_sum(s) == T(0) && lane == 0) v[c + 1] = kMark;
+    }
+}
+
 // QR of one matrix per workgroup, and with nrhs > 0 the least-squares
 // solution: the right-hand sides ride along as columns n .. n + nrhs - 1, so
 // the factorisation leaves Q^T b; R and those go to LDS and one wavefront
@@ -85,13 +105,16 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
         const T *src = (c >= n && c < n + nrhs) ? bb + (int64_t)(c - n) * ldb : a + (int64_t)(c < n ? c : 0) * lda;
         qr.load(q, src, m, c < n + nrhs);
     }
-    qr.factor(n, n + nrhs, vbuf, s_tau, taus, tau == nullptr && nrhs == 0);  // uniform
+    qr.factor(n, n + nrhs, vbuf, s_tau, taus);
 #pragma unroll
     for (int q = 0; q < SL; ++q) qr.store(q, a + (int64_t)qr.col(q) * lda, m, qr.col(q) < n);
     if (tau != nullptr)
         for (int i = threadIdx.x; i < n; i += NW * kWave) tau[b * strideTau + i] = taus[i];
     if (threadIdx.x == 0 && info != nullptr) info[b] = 0;
-    if (nrhs == 0) return;
+    if (nrhs == 0) {
+        if (tau == nullptr) mark_tails<T, NW>(a, lda, m, n, taus);  // uniform
+        return;
+    }
     T *R = reinterpret_cast<T *>(dyn_regs);
     const int ldr = n | 1;
 #pragma unroll
@@ -114,7 +137,7 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
 // few columns go one to a wavefront over as many workgroups as there are;
 // batches that fill the chip take four.  tau NULL: the scalar is formed from
 // the vector, tau = 2 / (1 + |v|^2), or 0 for |v|^2 = 0 (H = I): least squares has
-// no room to keep it between launches, and RegQr::reflect sees to it that no
+// no room to keep it between launches, and mark_tails sees to it that no
 // other reflector has |v|^2 = 0.  Only the first mout rows of C are
 // written (least squares leaves the rest of b as it was).
 constexpr int kOrmThreads = 256;

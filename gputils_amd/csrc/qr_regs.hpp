@@ -137,14 +137,7 @@ struct RegQr {
     // Reflector of column c (this wavefront's slot q): the column becomes
     // [R; beta; v], vb the vector [0 .. 0, 0, v] without its unit entry (with
     // it for kUnit = 0), *s_tau and tau[c] its scalar.
-    // keep: the scalar will be formed again from v (ormqr_regs_kernel), where
-    // |v|^2 = 0 stands for H = I.  A tail so small beside alpha that its square
-    // underflows has tau = 2 and beta = -alpha all the same, so the first entry
-    // of such a v becomes kMark: its square is a normal number, and it changes
-    // what the reflector does by kMark, far below the type's rounding.
-    static constexpr double kLost = sizeof(T) == 8 ? 0x1p-900 : 0x1p-120;  // |v|^2
-    static constexpr double kMark = sizeof(T) == 8 ? 0x1p-450 : 0x1p-60;
-    __device__ __forceinline__ void reflect(T (&xc)[KR], int c, T *vb, T *s_tau, T *tau, bool keep) {
+    __device__ __forceinline__ void reflect(T (&xc)[KR], int c, T *vb, T *s_tau, T *tau) {
         const int go = (c / NW) % kGroups;
         T asel = xc[0];
 #pragma unroll
@@ -168,12 +161,11 @@ struct RegQr {
             sc = 1.0;
         }
         const T scale = (T)sc;
-        const bool lost = keep && t != 0.0 && sc * (double)sq * sc < kLost;
         if (g == go) {
 #pragma unroll
             for (int k = 0; k < KR; ++k) {
                 const int i = l + LPC * k;
-                const T v = (lost && i == c + 1) ? (T)kMark : xc[k] * scale;
+                const T v = xc[k] * scale;
                 vb[i] = (i > c) ? v : ((kUnit == 0 && i == c) ? T(1) : T(0));
                 xc[k] = (i > c) ? v : ((i == c) ? (T)beta : xc[k]);
             }
@@ -271,9 +263,9 @@ struct RegQr {
     // reflector is read from LDS, the owner of the next column brings that
     // one up to date and forms the next reflector, the others update what
     // they hold; one barrier.  The owner's other columns wait until after the
-    // barrier, off the chain.  Ends with a barrier.  keep as in reflect.
-    __device__ __forceinline__ void factor(int n, int ntot, T *vbuf, T *s_tau, T *tau, bool keep = false) {
-        if (wave == 0) reflect(x[0], 0, vbuf, s_tau, tau, keep);
+    // barrier, off the chain.  Ends with a barrier.
+    __device__ __forceinline__ void factor(int n, int ntot, T *vbuf, T *s_tau, T *tau) {
+        if (wave == 0) reflect(x[0], 0, vbuf, s_tau, tau);
         __syncthreads();
         T vr[KR], t = T(0);
         int late = SL;  // slot formed in the last step: the others wait for its reflector's update
@@ -296,7 +288,7 @@ struct RegQr {
                 for (int q = 0; q < SL; ++q)
                     if (q == late) {
                         update_one(x[q], col(q), j, vr, t);  // columns past ntot hold zeros
-                        reflect(x[q], c1, vbuf + (c1 & 1) * kRows, s_tau + (c1 & 1), tau, keep);
+                        reflect(x[q], c1, vbuf + (c1 & 1) * kRows, s_tau + (c1 & 1), tau);
                     }
             } else {
                 update_all(SL, j, ntot, vr, t);
