@@ -329,25 +329,50 @@ __device__ __forceinline__ void hqr_factor(T *A, int64_t lda, int m, int n, T *t
     }
 }
 
+// The same without anything held in registers between rows: a reflector reads
+// and writes the rows from its own on and no others, and H = I (tau = 0) leaves
+// everything as it is.  For matrices with infinities or NaNs, where the zeros
+// that pad a reflector are not neutral.
+template <typename T, typename ACC, int NW>
+__device__ __forceinline__ void hqr_plain(T *A, int64_t lda, int m, int n, T *tau, T *s_tau) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int j = 0; j < n; ++j) {
+        if (wave == 0) {
+            const T t = make_reflector<T, ACC>(A, lda, m, j);
+            if (lane == 0) s_tau[0] = tau[j] = t;
+        }
+        __syncthreads();
+        const T t = s_tau[0];
+        if (t != T(0))
+            for (int c = j + 1 + wave; c < n; c += NW) apply_reflector_col<T, ACC>(A, lda, m, j, t, c);
+        __syncthreads();
+    }
+}
+
+// c <- (I - t v v^T) c for one m-vector in LDS, one wavefront, v = [1; v[j+1:m]]
+// from row j on; t = 0 leaves c as it is.
+template <typename T, typename ACC>
+__device__ __forceinline__ void apply_reflector_vec(const T *v, int m, int j, T t, T *c) {
+    if (t == T(0)) return;
+    const int lane = threadIdx.x & 63;
+    ACC w = ACC(0);
+    for (int i = j + 1 + lane; i < m; i += kWave) w += (ACC)v[i] * (ACC)c[i];
+    w = wave_sum(w) + (ACC)c[j];
+    const T tw = (T)((ACC)t * w);
+    for (int i = j + 1 + lane; i < m; i += kWave) c[i] -= tw * v[i];
+    wave_sync();
+    if (lane == 0) c[j] -= tw;
+    wave_sync();
+}
+
 // c <- Q^T c (trans) or Q c for one m-vector in LDS, one wavefront; Q from
 // the first k reflectors stored in A / tau.
 template <typename T, typename ACC>
 __device__ __forceinline__ void apply_q_vec(const T *A, int64_t lda, int m, int k, const T *tau, T *c,
                                             bool trans) {
-    const int lane = threadIdx.x & 63;
     for (int t = 0; t < k; ++t) {
         const int j = trans ? t : (k - 1 - t);
-        const T tj = tau[j];
-        if (tj == T(0)) continue;
-        const T *v = A + (int64_t)j * lda;
-        ACC w = ACC(0);
-        for (int i = j + 1 + lane; i < m; i += kWave) w += (ACC)v[i] * (ACC)c[i];
-        w = wave_sum(w) + (ACC)c[j];
-        const T tw = (T)((ACC)tj * w);
-        for (int i = j + 1 + lane; i < m; i += kWave) c[i] -= tw * v[i];
-        wave_sync();
-        if (lane == 0) c[j] -= tw;
-        wave_sync();
+        apply_reflector_vec<T, ACC>(A + (int64_t)j * lda, m, j, tau[j], c);
     }
 }
 

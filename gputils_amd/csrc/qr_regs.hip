@@ -61,6 +61,39 @@ __device__ __forceinline__ void trsv_regs(const T *R, int ldr, int n, T *c) {
     }
 }
 
+// The first n rows of Q^T b by one wavefront, lane i holding rows i + 64 u of b:
+// a reflector takes and changes the rows from its own on and no others, and H = I
+// none, so that an infinity or a NaN reaches no row that it should not.
+template <typename T, int U>
+__device__ __forceinline__ void qtb_plain(const T *A, int64_t lda, int m, int n, const T *tau, const T *b, T *c) {
+    const int lane = threadIdx.x & 63;
+    T y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) y[u] = (lane + kWave * u < m) ? b[lane + kWave * u] : T(0);
+#pragma unroll 1
+    for (int j = 0; j < n; ++j) {
+        const T t = tau[j];
+        if (t == T(0)) continue;
+        const T *v = A + (int64_t)j * lda;
+        T w = T(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = lane + kWave * u;
+            if (i >= j && i < m) w = fma(i == j ? T(1) : v[i], y[u], w);
+        }
+        w = t * wave_sum(w);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = lane + kWave * u;
+            if (i >= j && i < m) y[u] = fma(-w, i == j ? T(1) : v[i], y[u]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (lane + kWave * u < n) c[lane + kWave * u] = y[u];
+    hh::wave_sync();
+}
+
 // For reflectors whose scalars will be formed again from v (ormqr_regs_kernel),
 // where |v|^2 = 0 stands for H = I.  A tail so small beside alpha that its square
 // underflows has tau = 2 and beta = -alpha all the same: the first entry of such a
@@ -85,8 +118,20 @@ __device__ __forceinline__ void mark_tails(T *A, int64_t lda, int m, int n, cons
 // solution: the right-hand sides ride along as columns n .. n + nrhs - 1, so
 // the factorisation leaves Q^T b; R and those go to LDS and one wavefront
 // per right-hand side substitutes back.  tau may be NULL.
+// In the registers the rows above a reflector meet zeros of it, through which
+// infinities and NaNs reach rows that the reflector does not.  A column that
+// has met one is NaN throughout and so is its scalar: the matrix, still as it
+// was in memory, is then factorised again there (hh::hqr_plain).
+// Wavefronts per SIMD to leave registers for: what the column steps alone take,
+// by the 32-bit words of the columns.  Left to itself the compiler gives the
+// rare path above some more, and 8192 FP32 100 x 30 factorisations (66 registers
+// where 64 fit) take 153 us instead of 147.
+constexpr int qr_waves(int words) {
+    return words <= 14 ? 8 : words <= 16 ? 7 : words <= 20 ? 6 : words <= 24 ? 5 : words <= 32 ? 4 : words <= 48 ? 3 : words <= 64 ? 2 : 1;
+}
 template <typename T, int LPC, int NW, int KR, int SL>
-__global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nrhs, T *A, int64_t lda,
+__global__ __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(
+    qr_waves(KR *SL *(int)sizeof(T) / 4) > NW / 4 ? qr_waves(KR *SL *(int)sizeof(T) / 4) : (NW + 3) / 4))) void qr_regs_kernel(int m, int n, int nrhs, T *A, int64_t lda,
                                                             int64_t strideA, T *B, int64_t ldb, int64_t strideB,
                                                             T *tau, int64_t strideTau, int *info, int64_t batch) {
     using Q = RegQr<T, T, T, LPC, NW, KR, SL>;
@@ -106,6 +151,21 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
         qr.load(q, src, m, c < n + nrhs);
     }
     qr.factor(n, n + nrhs, vbuf, s_tau, taus);
+    bool odd = false;
+    for (int i = qr.lane; i < n; i += kWave) odd = odd || !__builtin_isfinite(taus[i]);
+    if (__builtin_expect(__any(odd), 0)) {  // the same in every wavefront
+        hh::hqr_plain<T, T, NW>(a, lda, m, n, taus, s_tau);
+        if (tau != nullptr)
+            for (int i = threadIdx.x; i < n; i += NW * kWave) tau[b * strideTau + i] = taus[i];
+        if (threadIdx.x == 0 && info != nullptr) info[b] = 0;
+        for (int r = qr.wave; r < nrhs; r += NW) {
+            T *rhs = bb + (int64_t)r * ldb, *c = reinterpret_cast<T *>(dyn_regs) + r * n;
+            qtb_plain<T, (Q::kRows + kWave - 1) / kWave>(a, lda, m, n, taus, rhs, c);
+            hh::trsv_upper<T>(a, lda, n, c);
+            for (int i = qr.lane; i < n; i += kWave) rhs[i] = c[i];
+        }
+        return;
+    }
 #pragma unroll
     for (int q = 0; q < SL; ++q) qr.store(q, a + (int64_t)qr.col(q) * lda, m, qr.col(q) < n);
     if (tau != nullptr)
@@ -122,6 +182,9 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
     __syncthreads();
     for (int r = qr.wave; r < nrhs; r += NW) {
         T *c = R + (n + r) * ldr;
+        bool spread = false;  // an infinity or a NaN in Q^T b
+        for (int i = qr.lane; i < n; i += kWave) spread = spread || !__builtin_isfinite(c[i]);
+        if (__builtin_expect(__any(spread), 0)) qtb_plain<T, (Q::kRows + kWave - 1) / kWave>(a, lda, m, n, taus, bb + (int64_t)r * ldb, c);
         if (n <= kWave) trsv_regs<T, 1>(R, ldr, n, c);
         else trsv_regs<T, 2>(R, ldr, n, c);
         hh::wave_sync();
@@ -138,7 +201,8 @@ __global__ __launch_bounds__(NW *kWave) void qr_regs_kernel(int m, int n, int nr
 // batches that fill the chip take four.  tau NULL: the scalar is formed from
 // the vector, tau = 2 / (1 + |v|^2), or 0 for |v|^2 = 0 (H = I): least squares has
 // no room to keep it between launches, and mark_tails sees to it that no
-// other reflector has |v|^2 = 0.  Only the first mout rows of C are
+// other reflector has |v|^2 = 0.  Columns that come out with an infinity or a
+// NaN are done again through LDS (see qr_regs_kernel).  Only the first mout rows of C are
 // written (least squares leaves the rest of b as it was).
 constexpr int kOrmThreads = 256;
 constexpr int kOrmWaves = kOrmThreads / kWave;
@@ -276,6 +340,34 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
         __syncthreads();
     }
     swap0(head);
+    bool odd = false;
+#pragma unroll
+    for (int s = 0; s < SL; ++s) odd = odd || !__builtin_isfinite(x[s][0]);
+    if (__builtin_expect(__any(odd), 0)) {
+        T *c = V[wave];  // this wavefront's own row; the last reflectors are past
+        for (int s = c0; s < c0 + SL && s < ncols; ++s) {
+            T *dst = cb + (int64_t)s * ldc;
+            for (int i = lane; i < m; i += kWave) c[i] = dst[i];
+            hh::wave_sync();
+            for (int e = 0; e < k; ++e) {
+                const int j = trans ? e : k - 1 - e;
+                const T *v = a + (int64_t)j * lda;
+                T t;
+                if (tau != nullptr) {
+                    t = tb[j];
+                } else {
+                    t = T(0);
+                    for (int i = j + 1 + lane; i < m; i += kWave) t = fma(v[i], v[i], t);
+                    t = wave_sum(t);
+                    t = (t == T(0)) ? T(0) : T(2) / (T(1) + t);
+                }
+                hh::apply_reflector_vec<T, T>(v, m, j, t, c);
+            }
+            for (int i = lane; i < mout; i += kWave) dst[i] = c[i];
+            hh::wave_sync();
+        }
+        return;
+    }
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
         if (c0 + s >= ncols) continue;

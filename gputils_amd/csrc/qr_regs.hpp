@@ -157,7 +157,7 @@ struct RegQr {
         else hh::reflector_scalars<float, double>((double)alpha, (double)sq, beta, t, sc);
         if (sq == ACC(0)) {  // H = I (dlarfg with x = 0): the column stays as it is
             beta = (double)alpha;
-            t = 0.0;
+            t = 0.0 * fabs((double)alpha);  // NaN for a column that has met an infinity or a NaN
             sc = 1.0;
         }
         const T scale = (T)sc;
