@@ -154,6 +154,7 @@ __global__ __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(
     bool odd = false;
     for (int i = qr.lane; i < n; i += kWave) odd = odd || !__builtin_isfinite(taus[i]);
     if (__builtin_expect(__any(odd), 0)) {  // the same in every wavefront
+        __syncthreads();  // all have read taus before it is formed again
         hh::hqr_plain<T, T, NW>(a, lda, m, n, taus, s_tau);
         if (tau != nullptr)
             for (int i = threadIdx.x; i < n; i += NW * kWave) tau[b * strideTau + i] = taus[i];
