@@ -376,6 +376,16 @@ __device__ __forceinline__ void apply_q_vec(const T *A, int64_t lda, int m, int 
     }
 }
 
+// Whether the reciprocal of d is a normal number: a substitution that multiplies
+// by it is as exact as a division only then (1 / d is infinite for the smaller
+// half of the subnormal d and has lost bits for the largest d).
+template <typename T>
+__device__ __forceinline__ bool has_reciprocal(T d) {
+    constexpr T lo = sizeof(T) == 8 ? T(0x1p-1022) : T(0x1p-126);
+    constexpr T hi = sizeof(T) == 8 ? T(0x1p+1022) : T(0x1p+126);
+    return fabs(d) >= lo && fabs(d) <= hi;
+}
+
 // Solve R y = c in place (R upper triangular n x n at A, c in LDS), one
 // wavefront, column-oriented back substitution.
 template <typename T>

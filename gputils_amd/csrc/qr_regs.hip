@@ -19,17 +19,24 @@ namespace qrr {
 
 // Back substitution R y = c by one wavefront: lane i holds rows i + 64 u of c
 // and the reciprocals of R's diagonal, column k - 1 of R (LDS, ld ldr) is
-// read while step k runs.
+// read while step k runs.  Where one has no normal reciprocal it divides.
 template <typename T, int NR>
 __device__ __forceinline__ void trsv_regs(const T *R, int ldr, int n, T *c) {
     const int lane = threadIdx.x & 63;
     T cv[NR], di[NR], rk[NR];
+    bool divide = false;
 #pragma unroll
     for (int u = 0; u < NR; ++u) {
         const int i = lane + kWave * u;
         cv[u] = (i < n) ? c[i] : T(0);
-        di[u] = (i < n) ? T(1) / R[i + i * ldr] : T(0);
+        di[u] = (i < n) ? R[i + i * ldr] : T(1);
+        divide = divide || !hh::has_reciprocal(di[u]);
+        di[u] = T(1) / di[u];
         rk[u] = (i < n) ? R[i + (n - 1) * ldr] : T(0);
+    }
+    if (__builtin_expect(__any(divide), 0)) {
+        hh::trsv_upper<T>(R, ldr, n, c);
+        return;
     }
 #pragma unroll 1
     for (int k = n - 1; k >= 0; --k) {
@@ -386,7 +393,8 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
 // diagonal; the workgroup's four share R, staged through LDS 16 columns at a
 // time with the next ones on their way.  A step is a broadcast, a product and
 // NU FMAs (about 90 cycles), where reading R's column from global memory in
-// every step made it 900: n = 150 in FP64, one column, 59 -> 20 us.
+// every step made it 900: n = 150 in FP64, one column, 59 -> 20 us.  Where a
+// diagonal entry has no normal reciprocal it divides, with R in memory.
 constexpr int kTrsmCols = 16;
 template <typename T, int NU>
 __global__ __launch_bounds__(kOrmThreads) void trsm_regs_kernel(int n, int nrhs, const T *R, int64_t ldr,
@@ -402,11 +410,24 @@ __global__ __launch_bounds__(kOrmThreads) void trsm_regs_kernel(int n, int nrhs,
     const bool ok = col < nrhs;
     T *x = B + b * strideB + (int64_t)(ok ? col : 0) * ldb;
     T c[NU], di[NU];
+    bool divide = false;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
         const int i = lane + kWave * u;
         c[u] = (i < n) ? x[i] : T(0);
-        di[u] = (i < n) ? T(1) / r[i + (int64_t)i * ldr] : T(0);
+        di[u] = (i < n) ? r[i + (int64_t)i * ldr] : T(1);
+        divide = divide || !hh::has_reciprocal(di[u]);
+        di[u] = T(1) / di[u];
+    }
+    if (__builtin_expect(__any(divide), 0)) {  // the same in every wavefront
+        T *y = S[wave];  // n <= kRows
+        if (ok) {
+            for (int i = lane; i < n; i += kWave) y[i] = x[i];
+            hh::wave_sync();
+            hh::trsv_upper<T>(r, ldr, n, y);
+            for (int i = lane; i < n; i += kWave) x[i] = y[i];
+        }
+        return;
     }
     // columns 16 q .. 16 q + 15; wavefront w stages four of them
     constexpr int kPer = kTrsmCols / kOrmWaves;
