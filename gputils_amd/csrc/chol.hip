@@ -116,6 +116,23 @@ __device__ __forceinline__ void pivot(double d, double &s, double &inv) {
     inv = tiny ? q * 0x1p+128 : q;
 }
 
+// The same for every positive d: v_rsq_f32 takes a subnormal d for zero, and for
+// an infinite one (a variable fixed by a penalty) s is infinite and inv zero,
+// where the steps above make NaNs.
+__device__ __forceinline__ void pivot_any(float d, float &s, float &inv) {
+    const bool tiny = d < 0x1p-126f;
+    const float dd = tiny ? d * 0x1p+48f : d;
+    const float q = __builtin_amdgcn_rsqf(dd);  // 0 for infinity
+    inv = tiny ? q * 0x1p+24f : q;
+    s = __builtin_isinf(d) ? d : (tiny ? dd * q * 0x1p-24f : d * inv);
+}
+__device__ __forceinline__ void pivot_any(double d, double &s, double &inv) {
+    pivot(d, s, inv);
+    const bool inf = __builtin_isinf(d);
+    inv = inf ? 0.0 : inv;
+    s = inf ? d : s;
+}
+
 // d += (v of lane LANE of the 16-lane row) * w: the FMA takes the other
 // lane's value by DPP (row_newbcast, the control that 64-bit arithmetic
 // takes), where readlane and an FMA would be three instructions in FP64.
@@ -199,14 +216,28 @@ __device__ __forceinline__ void tri_inverse_steps(const T (&row)[16], T dinv, T 
     }
 }
 
+// Whether d is not a positive normal number: 1 or 0 from its bits, as d is
+// uniform and the scalar unit has time beside the pivots' chain.
+__device__ __forceinline__ unsigned unusual(float d) {
+    return (unsigned)__float_as_int(d) - 0x00800000u >= 0x7f000000u;
+}
+__device__ __forceinline__ unsigned unusual(double d) {
+    return (unsigned)(__double_as_longlong(d) >> 32) - 0x00100000u >= 0x7fe00000u;
+}
+
 // Steps K.. of the factorisation of a 16x16 block (see factor_diag_block).
-template <int K, typename T>
+// PIV: kNormal and kAny take pivot or pivot_any and leave the first failing
+// step in `fail`; kWatch takes pivot and leaves whether a d was unusual.
+constexpr int kNormal = 0, kAny = 1, kWatch = 2;
+template <int PIV, int K, typename T>
 __device__ __forceinline__ void factor_steps(T (&row)[16], T (&nx)[16], int lane, int &fail) {
     if constexpr (K < 16) {
         const T d = readlane(row[K], K);
-        if (fail < 0 && !(d > T(0))) fail = K;  // uniform; also catches NaN
+        if constexpr (PIV == kWatch) fail |= unusual(d);
+        else if (fail < 0 && !(d > T(0))) fail = K;  // uniform; also catches NaN
         T sq, inv;
-        pivot(d, sq, inv);
+        if constexpr (PIV == kAny) pivot_any(d, sq, inv);
+        else pivot(d, sq, inv);
         const T lk = ((lane & 15) == K) ? sq : row[K] * inv;
         row[K] = lk;
         const T nl = -lk;
@@ -223,7 +254,7 @@ __device__ __forceinline__ void factor_steps(T (&row)[16], T (&nx)[16], int lane
         // left to the compiler, every row's readlane results were hoisted
         // into SGPRs and spilled
         asm volatile("" : "+v"(nx[K]));
-        factor_steps<K + 1>(row, nx, lane, fail);
+        factor_steps<PIV, K + 1>(row, nx, lane, fail);
     }
 }
 
@@ -244,7 +275,10 @@ __device__ __forceinline__ void factor_steps(T (&row)[16], T (&nx)[16], int lane
 // spreads are never stored), so the pivot chain of column k + 1 overlaps
 // the rest of step k.  Entries above the diagonal are updated with garbage
 // and never read: only lanes r > j read row[j].
-template <typename T>
+// ANY: pivots of the whole range of the type, for n > 128.  The 16 steps are
+// done again with pivot_any where one was not a positive normal number (with it
+// in all of them a block would take 20 % longer in FP32).
+template <bool ANY = false, typename T>
 __device__ __forceinline__ int factor_diag_block(T *blk, T *Lout, int64_t ldo, int nvalid) {
     // a lane index the compiler cannot relate to the one of the other
     // phases, so the per-step lane masks below are formed where they are
@@ -255,7 +289,17 @@ __device__ __forceinline__ int factor_diag_block(T *blk, T *Lout, int64_t ldo, i
 #pragma unroll
     for (int c = 0; c < 16; ++c) row[c] = blk[sw(lane & 15, c)];
     int fail = -1;
-    factor_steps<0>(row, nx, lane, fail);
+    if constexpr (ANY) {
+        int odd = 0;
+        factor_steps<kWatch, 0>(row, nx, lane, odd);
+        if (__builtin_expect(odd, 0)) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) row[c] = blk[sw(lane & 15, c)];
+            factor_steps<kAny, 0>(row, nx, lane, fail);
+        }
+    } else {
+        factor_steps<kNormal, 0>(row, nx, lane, fail);
+    }
     if (fail >= 0) return fail;
     if (Lout != nullptr && lane < nvalid) {
 #pragma unroll
@@ -590,8 +634,9 @@ constexpr int64_t kStripMaxN = 16 * kStripWorkers * kStripSlots;
 static_assert(kStripMaxN <= 2 * kStripThreads, "potrs_strips_kernel holds two rows a thread");
 constexpr int64_t kStripMaxLd = 1 << 26;  // lane offsets of up to 13 columns are 32-bit
 
+// Two strips in FP64 fit the registers of two workgroups per CU.
 template <typename T, int S>
-__global__ __launch_bounds__(kStripThreads) void potrf_strips_kernel(int n, T *A, int64_t lda, int64_t strideA,
+__global__ __launch_bounds__(kStripThreads) __attribute__((amdgpu_waves_per_eu(S == 2 ? 4 : 2))) void potrf_strips_kernel(int n, T *A, int64_t lda, int64_t strideA,
                                                                      int *info, int64_t batch) {
     using M = Mfma16<T>;
     __shared__ T dg[2][256];  // diagonal block J, then its inverse (slot J & 1)
@@ -613,7 +658,7 @@ __global__ __launch_bounds__(kStripThreads) void potrf_strips_kernel(int n, T *A
         int fail = 0;
 #pragma unroll 1
         for (int J = 0; J < nb; ++J) {
-            const int f = factor_diag_block(dg[J & 1], a + 16 * J + (int64_t)16 * J * lda, lda, n - 16 * J);
+            const int f = factor_diag_block<true>(dg[J & 1], a + 16 * J + (int64_t)16 * J * lda, lda, n - 16 * J);
             fail = (f >= 0) ? 16 * J + f + 1 : 0;  // uniform
             if (lane == 0) s_flag = fail;
             __syncthreads();
@@ -742,6 +787,35 @@ __global__ __launch_bounds__(kStripThreads) void potrf_strips_kernel(int n, T *A
     }
 }
 
+// L L^T x = b by columns for each right-hand side, one workgroup of NT threads;
+// red: NT elements of LDS.
+template <int NT, typename T>
+__device__ __forceinline__ void substitute(int n, int nrhs, const T *l, int64_t lda, T *B, int64_t ldb, T *red) {
+    for (int r = 0; r < nrhs; ++r) {
+        T *x = B + (int64_t)r * ldb;
+        for (int k = 0; k < n; ++k) {
+            __syncthreads();
+            const T xk = x[k] / l[k + (int64_t)k * lda];
+            __syncthreads();
+            if (threadIdx.x == 0) x[k] = xk;
+            for (int i = k + 1 + threadIdx.x; i < n; i += NT) x[i] -= l[i + (int64_t)k * lda] * xk;
+        }
+        for (int k = n - 1; k >= 0; --k) {
+            __syncthreads();
+            // x_k = (x_k - sum_{i>k} l_ik x_i) / l_kk : block reduction
+            T part = T(0);
+            for (int i = k + 1 + threadIdx.x; i < n; i += NT) part += l[i + (int64_t)k * lda] * x[i];
+            red[threadIdx.x] = part;
+            __syncthreads();
+            for (int s = NT / 2; s > 0; s >>= 1) {
+                if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+                __syncthreads();
+            }
+            if (threadIdx.x == 0) x[k] = (x[k] - red[0]) / l[k + (int64_t)k * lda];
+        }
+    }
+}
+
 // Solve with the factor of a larger matrix (n in (128, kStripMaxN]) for any
 // nrhs, four right-hand sides per pass.  The reference substitution is a
 // chain of 2 n dependent steps; here the diagonal blocks are inverted first
@@ -757,6 +831,8 @@ __global__ __launch_bounds__(kStripThreads) void potrf_strips_kernel(int n, T *A
 // 47 us now.
 // skip != nullptr: systems with skip[b] != 0 (a failed factorisation) are
 // left as they are, as LAPACK dposv leaves B.
+// A factor with a diagonal entry that has no normal reciprocal is substituted
+// by columns, with divisions.
 // ROWS: rows of a thread, n <= ROWS * kStripThreads.
 template <typename T, int ROWS>
 __global__ __launch_bounds__(kStripThreads) void potrs_strips_kernel(int n, int nrhs, const T *L, int64_t lda,
@@ -775,21 +851,34 @@ __global__ __launch_bounds__(kStripThreads) void potrs_strips_kernel(int n, int 
     T *Y = D + 256 * nb;                       // npad x 4
     T *Z = Y + npad * kRhsChunk;               // 16 x 4 sums of the backward step
     const T *l = L + b * strideL;
+    bool divide = false;
     for (int J = wave; J < nb; J += kStripWaves) {
         T row[16], nx[16];
         const int gi = 16 * J + c;
 #pragma unroll
         for (int k = 0; k < 16; ++k)
             row[k] = (gi < n && c >= k) ? l[gi + (int64_t)(16 * J + k) * lda] : ((c == k) ? T(1) : T(0));
-        tri_inverse_steps<0>(row, (gi < n) ? T(1) / l[gi + (int64_t)gi * lda] : T(1), nx);
+        const T d = (gi < n) ? l[gi + (int64_t)gi * lda] : T(1);
+        divide = divide || !hh::has_reciprocal(d);
+        tri_inverse_steps<0>(row, T(1) / d, nx);
         if (lane < 16) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) D[256 * J + sw(r, lane)] = -nx[r];
         }
     }
     T *bb = B + b * strideB;
-    for (int r0 = 0; r0 < nrhs; r0 += kRhsChunk) {
+    int *flag = reinterpret_cast<int *>(Z);  // one for each wavefront
+    divide = __any(divide);
+    if (lane == 0) flag[wave] = divide;
+    __syncthreads();
+    if (__builtin_expect(__any(lane < kStripWaves && flag[lane]), 0)) {  // the same in every wavefront
         __syncthreads();
+        substitute<kStripThreads>(n, nrhs, l, lda, bb, ldb, D);  // 256 nb > kStripThreads
+        if (threadIdx.x == 0 && info != nullptr) info[b] = 0;
+        return;
+    }
+    for (int r0 = 0; r0 < nrhs; r0 += kRhsChunk) {
+        if (r0 > 0) __syncthreads();
         for (int e = threadIdx.x; e < npad * kRhsChunk; e += kStripThreads) {
             const int row = e % npad, col = e / npad;
             Y[e] = (row < n && r0 + col < nrhs) ? bb[row + (int64_t)(r0 + col) * ldb] : T(0);
@@ -951,31 +1040,8 @@ __global__ __launch_bounds__(kThreads) void potrs_global_kernel(int n, int nrhs,
     const int64_t b = blockIdx.x;
     if (b >= batch) return;
     if (skip != nullptr && skip[b] != 0) return;
-    const T *l = L + b * strideL;
-    for (int r = 0; r < nrhs; ++r) {
-        T *x = B + b * strideB + (int64_t)r * ldb;
-        for (int k = 0; k < n; ++k) {
-            __syncthreads();
-            const T xk = x[k] / l[k + (int64_t)k * lda];
-            __syncthreads();
-            if (threadIdx.x == 0) x[k] = xk;
-            for (int i = k + 1 + threadIdx.x; i < n; i += kThreads) x[i] -= l[i + (int64_t)k * lda] * xk;
-        }
-        for (int k = n - 1; k >= 0; --k) {
-            __syncthreads();
-            // x_k = (x_k - sum_{i>k} l_ik x_i) / l_kk : block reduction
-            __shared__ T red[kThreads];
-            T part = T(0);
-            for (int i = k + 1 + threadIdx.x; i < n; i += kThreads) part += l[i + (int64_t)k * lda] * x[i];
-            red[threadIdx.x] = part;
-            __syncthreads();
-            for (int s = kThreads / 2; s > 0; s >>= 1) {
-                if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-                __syncthreads();
-            }
-            if (threadIdx.x == 0) x[k] = (x[k] - red[0]) / l[k + (int64_t)k * lda];
-        }
-    }
+    __shared__ T red[kThreads];
+    substitute<kThreads>(n, nrhs, L + b * strideL, lda, B + b * strideB, ldb, red);
     if (threadIdx.x == 0 && info != nullptr) info[b] = 0;
 }
 
