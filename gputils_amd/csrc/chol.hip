@@ -301,7 +301,7 @@ __device__ __forceinline__ int factor_diag_block(T *blk, T *Lout, int64_t ldo, i
         factor_steps<kNormal, 0>(row, nx, lane, fail);
     }
     if (fail >= 0) return fail;
-    if (Lout != nullptr && lane < nvalid) {
+    if (Lout != nullptr && lane < 16 && lane < nvalid) {  // the rows below belong to others
 #pragma unroll
         for (int c = 0; c < 16; ++c)
             if (c <= lane && c < nvalid) Lout[lane + (int64_t)c * ldo] = row[c];
