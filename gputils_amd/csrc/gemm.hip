@@ -223,23 +223,45 @@ __global__ __launch_bounds__(64 * WV *WV) __attribute__((amdgpu_waves_per_eu(4))
             put(smem[cur ^ (kBufs - 1)]);
             __syncthreads();
         }
-        multiply(smem[cur], k - k0);
+        // entry e of tile (y, x) of this lane, and whether it lies in C
+        auto each = [&](auto f) {
 #pragma unroll
-        for (int y = 0; y < NY; ++y)
+            for (int y = 0; y < NY; ++y)
 #pragma unroll
-            for (int x = 0; x < NX; ++x) {
-                const int gi = i0 + wm + 16 * x + r;
+                for (int x = 0; x < NX; ++x) {
+                    const int gi = i0 + wm + 16 * x + r;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int gj = j0 + wn + 16 * y + M::drow(lane, e);
-                    if (gi < m && gj < n) {
-                        T *dst = c + gi + (int64_t)gj * ldc;
-                        T v = alpha * acc[y][x][e];
-                        if (beta != T(0)) v += beta * *dst;
-                        *dst = v;
+                    for (int e = 0; e < 4; ++e) {
+                        const int gj = j0 + wn + 16 * y + M::drow(lane, e);
+                        if (gi < m && gj < n) f(y, x, e, c + gi + (int64_t)gj * ldc);
                     }
                 }
-            }
+        };
+        if (WV == 1) {  // short of registers: 16384 FP32 16 x 17 x 4 23 us, with the reads first 28
+            multiply(smem[cur], k - k0);
+            each([&](int y, int x, int e, T *dst) {
+                T v = alpha * acc[y][x][e];
+                if (beta != T(0)) v += beta * *dst;
+                *dst = v;
+            });
+            return;
+        }
+        if (beta == T(0)) {
+            multiply(smem[cur], k - k0);
+            each([&](int y, int x, int e, T *dst) { *dst = alpha * acc[y][x][e]; });
+            return;
+        }
+        // C is read as a whole while the last chunk is multiplied: an entry at a
+        // time, each load would wait for the store before it (8738 FP32 100 x 33
+        // x 1 126 us, so 93)
+        T old[NY > 0 ? NY : 1][NX > 0 ? NX : 1][4];
+        each([&](int y, int x, int e, const T *src) { old[y][x][e] = *src; });
+        multiply(smem[cur], k - k0);
+        each([&](int y, int x, int e, T *dst) {
+            T v = alpha * acc[y][x][e];
+            v += beta * old[y][x][e];
+            *dst = v;
+        });
     };
     using Zero = std::integral_constant<int, 0>;
     using One = std::integral_constant<int, 1>;
