@@ -342,8 +342,8 @@ class RaggedLeastSquares:
         return [dict(zip(keys, desc[7 * i:7 * i + 7])) for i in range(nb.value)]
 
     def configure(self, bucket: int, method: int, waves: int, per_cu: int, queue: int = 0):
-        """Set one bucket's launch shape: method 0 (column steps in LDS,
-        waves 2/4/8/16) or 1 (register panels, waves 8/16), workgroups per
+        """Set one bucket's launch shape: method 0 (columns in registers one
+        by one, waves 2/4/8/16) or 1 (in panels, waves 8/16), workgroups per
         CU, static ranges (queue 0) or a work queue (queue 1)."""
         check(lib().gputils_gels_ragged_plan_configure(self._plan, bucket, method, waves, per_cu, queue),
               "plan_configure")

@@ -473,14 +473,19 @@ __device__ __forceinline__ void ragged_factor(const double *__restrict__ a, cons
     }
 }
 
-// Wavefronts per SIMD to leave registers for: in the smaller buckets one
-// register too many (129 where 128 fit) costs a workgroup per CU, 1089 against
-// 1065 us for 4096 systems of 8 to 64 columns.
-constexpr int ragged_waves(int maxe, int nw, int method) {
+// Wavefronts per SIMD to leave registers for.  In the smaller buckets one
+// register too many (129 where 128 fit) costs a workgroup per CU; so does the
+// compiler's own choice for eight wavefronts in the 8 K bucket (153 with no
+// spill, 128 with 5 in scratch): alone on its CU a workgroup has nothing beside
+// the single wavefronts of its solves and refinement steps, and 4096 systems of
+// 64 columns, two steps, took 2100 us, with two workgroups 1512 (with the
+// columns in LDS, 2061).
+// MANY: for the 16 K bucket with more workgroups than CUs, see launch_ragged_one.
+constexpr int ragged_waves(int maxe, int nw, int method, bool many) {
     const int least = nw < 4 ? 1 : nw / 4;
     if (method != 0) return least;
     const int fit = maxe == 2048 ? (nw == 2 ? 3 : 4) : maxe == 4096 ? (nw >= 8 ? 4 : nw == 4 ? 3 : 2)
-                  : maxe == 8192 ? (nw == 8 ? 3 : nw == 4 ? 2 : 1) : 1;
+                  : maxe == 8192 ? (nw == 8 ? 4 : nw == 4 ? 2 : 1) : maxe == 16384 && many ? 4 : 1;
     return fit > least ? fit : least;
 }
 
@@ -509,8 +514,8 @@ constexpr int ragged_waves(int maxe, int nw, int method) {
 // arithmetic is the same for every NW and every item-to-workgroup
 // assignment, so the results are too; the two methods round the FP32
 // factorisation differently.
-template <int MAXE, int NW, int METHOD>
-__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(ragged_waves(MAXE, NW, METHOD)))) void gels_ragged_kernel(const RaggedItem *__restrict__ items,
+template <int MAXE, int NW, int METHOD, bool MANY>
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(ragged_waves(MAXE, NW, METHOD, MANY)))) void gels_ragged_kernel(const RaggedItem *__restrict__ items,
                                                                const int *__restrict__ wstart,
                                                                const double *__restrict__ A, double *B,
                                                                int steps, int *queue) {
@@ -645,37 +650,46 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(ragg
 
 // Launch one bucket of a ragged plan: the LDS capacity MAXE, the
 // factorisation method and the wavefronts per workgroup pick the
-// instantiation.
+// instantiation.  In the 16 K bucket eight wavefronts hold 193 registers a lane,
+// one workgroup per CU, or with 92 of them in scratch 128 and two.  Up to as
+// many workgroups as CUs the first is faster (256 systems of 32 to 50 columns
+// and 260 to 320 rows, one step: 97 us, the other 132); beyond, the second
+// fills the solves and refinement steps of one workgroup with another's columns
+// (2000 systems of 64 columns and 129 to 255 rows, two steps: 1159 against 730;
+// columns in LDS, 1015), but not without such a step.
 template <int MAXE, int METHOD, int NW>
 void launch_ragged_one(int grid, hipStream_t st, const RaggedItem *items, const int *wstart, const double *A,
-                       double *B, int steps, int *queue) {
-    hipLaunchKernelGGL((gels_ragged_kernel<MAXE, NW, METHOD>), dim3(grid), dim3(NW * kWave), 0, st, items, wstart, A,
-                       B, steps, queue);
+                       double *B, int steps, int *queue, int cus) {
+    auto kern = gels_ragged_kernel<MAXE, NW, METHOD, false>;
+    if constexpr (MAXE == 16384 && METHOD == 0 && NW == 8)
+        if (grid > cus && steps > 0) kern = gels_ragged_kernel<MAXE, NW, METHOD, true>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * kWave), 0, st, items, wstart, A, B, steps, queue);
 }
 
 template <int MAXE>
 void launch_ragged_maxe(int method, int waves, int grid, hipStream_t st, const RaggedItem *items, const int *wstart,
-                        const double *A, double *B, int steps, int *queue) {
+                        const double *A, double *B, int steps, int *queue, int cus) {
     if (method == 1) {
-        if (waves == 16) launch_ragged_one<MAXE, 1, 16>(grid, st, items, wstart, A, B, steps, queue);
-        else launch_ragged_one<MAXE, 1, 8>(grid, st, items, wstart, A, B, steps, queue);
+        if (waves == 16) launch_ragged_one<MAXE, 1, 16>(grid, st, items, wstart, A, B, steps, queue, cus);
+        else launch_ragged_one<MAXE, 1, 8>(grid, st, items, wstart, A, B, steps, queue, cus);
     } else {
-        if (waves == 2) launch_ragged_one<MAXE, 0, 2>(grid, st, items, wstart, A, B, steps, queue);
-        else if (waves == 4) launch_ragged_one<MAXE, 0, 4>(grid, st, items, wstart, A, B, steps, queue);
-        else if (waves == 16) launch_ragged_one<MAXE, 0, 16>(grid, st, items, wstart, A, B, steps, queue);
-        else launch_ragged_one<MAXE, 0, 8>(grid, st, items, wstart, A, B, steps, queue);
+        if (waves == 2) launch_ragged_one<MAXE, 0, 2>(grid, st, items, wstart, A, B, steps, queue, cus);
+        else if (waves == 4) launch_ragged_one<MAXE, 0, 4>(grid, st, items, wstart, A, B, steps, queue, cus);
+        else if (waves == 16) launch_ragged_one<MAXE, 0, 16>(grid, st, items, wstart, A, B, steps, queue, cus);
+        else launch_ragged_one<MAXE, 0, 8>(grid, st, items, wstart, A, B, steps, queue, cus);
     }
 }
 
-// queue: NULL for the static ranges, else the bucket's two counters
+// queue: NULL for the static ranges, else the bucket's two counters; cus: of
+// the plan's device
 int launch_ragged(int maxe, int method, int waves, int grid, hipStream_t st, const RaggedItem *items,
-                  const int *wstart, const double *A, double *B, int steps, int *queue) {
+                  const int *wstart, const double *A, double *B, int steps, int *queue, int cus) {
     switch (maxe) {
-    case 2048: launch_ragged_maxe<2048>(method, waves, grid, st, items, wstart, A, B, steps, queue); break;
-    case 4096: launch_ragged_maxe<4096>(method, waves, grid, st, items, wstart, A, B, steps, queue); break;
-    case 8192: launch_ragged_maxe<8192>(method, waves, grid, st, items, wstart, A, B, steps, queue); break;
-    case 16384: launch_ragged_maxe<16384>(method, waves, grid, st, items, wstart, A, B, steps, queue); break;
-    default: launch_ragged_maxe<32768>(method, waves, grid, st, items, wstart, A, B, steps, queue); break;
+    case 2048: launch_ragged_maxe<2048>(method, waves, grid, st, items, wstart, A, B, steps, queue, cus); break;
+    case 4096: launch_ragged_maxe<4096>(method, waves, grid, st, items, wstart, A, B, steps, queue, cus); break;
+    case 8192: launch_ragged_maxe<8192>(method, waves, grid, st, items, wstart, A, B, steps, queue, cus); break;
+    case 16384: launch_ragged_maxe<16384>(method, waves, grid, st, items, wstart, A, B, steps, queue, cus); break;
+    default: launch_ragged_maxe<32768>(method, waves, grid, st, items, wstart, A, B, steps, queue, cus); break;
     }
     return launch_check("gels_ragged_kernel");
 }
@@ -735,7 +749,7 @@ struct gputils_gels_plan {
         int maxe;
         int begin, count;  // items begin .. begin + count - 1 of d_items
         int wbase;         // first of this bucket's count + 1 slots in d_wstart
-        int method;        // factorisation: 0 column steps in LDS, 1 register panels
+        int method;        // factorisation: 0 columns in registers one by one, 1 in panels
         int waves;         // wavefronts per workgroup: 2, 4, 8, 16 (method 0) or 8, 16 (method 1)
         int per_cu;        // workgroups per CU the grid is sized for
         int grid;          // min(count, CUs * per_cu)
@@ -771,14 +785,20 @@ constexpr int kRaggedBuckets = 5;
 // c 2048, h 256, dx 256, xd 512, rd 4096, bd 4096 bytes)
 int ragged_lds_bytes(int maxe) { return (maxe + 512) * 4 + 11536; }
 
-// most workgroups of one bucket that a CU can hold at once: LDS (160 KiB)
-// and 32 wavefronts per CU
+// Most workgroups per CU that a bucket is launched with, or tuned to: what the
+// LDS (160 KiB) and 32 wavefronts hold.  The registers of method 0 leave fewer of
+// them resident (with eight wavefronts two in the 2, 4 and 8 K buckets and one
+// or two in the 16 K one), and the ranges of the others follow as those end.
+// Grids of the resident number alone are no better: a static range's cost is an
+// estimate, and more, shorter ranges even it out (over 16 sets of systems and 0
+// to 2 steps 4 % slower in the mean; 4096 systems of 30 to 50 columns, two
+// steps, 1008 us instead of 848).
 int ragged_max_per_cu(int maxe, int waves) {
     return std::max(1, std::min(160 * 1024 / ragged_lds_bytes(maxe), 32 / waves));
 }
 
 // estimated cost of one system: the factorisation's m n^2 work spread over
-// a wavefront plus the n-step serial chains of the solves
+// a wavefront plus the n-step serial chains of reflectors and solves
 double ragged_cost(int m, int n) { return (double)m * n * n / 64.0 + 2000.0 * n; }
 
 // Assign the bucket's items to its grid (longest processing time first:
@@ -838,7 +858,8 @@ int ragged_execute(gputils_gels_plan *plan, const double *A, double *B, int step
         hipStream_t sb = (conc && b > 0) ? plan->streams[b - 1] : st;
         if (conc && b > 0) GPUTILS_HIP(hipStreamWaitEvent(sb, plan->fork, 0));
         int rc = qr::launch_ragged(bk.maxe, bk.method, bk.waves, bk.grid, sb, plan->d_items,
-                                   plan->d_wstart + bk.wbase, A, B, steps, bk.queue ? plan->d_queue + 2 * b : nullptr);
+                                   plan->d_wstart + bk.wbase, A, B, steps, bk.queue ? plan->d_queue + 2 * b : nullptr,
+                                   plan->cus);
         if (rc) return rc;
         if (conc && b > 0) GPUTILS_HIP(hipEventRecord(plan->done[b - 1], sb));
     }
@@ -993,8 +1014,8 @@ int gputils_gels_ragged_plan_create(gputils_gels_plan_t *plan, int64_t count, co
         b.count = (int)mem.size();
         b.wbase = begin + (int)p->buckets.size();
         b.order = std::move(mem);
-        // untuned shape: column steps, eight wavefronts, as many workgroups
-        // per CU as fit
+        // untuned shape: columns one by one, eight wavefronts, as many
+        // workgroups per CU as LDS and wavefronts allow
         ragged_set_shape(p, b, 0, 8, ragged_max_per_cu(b.maxe, 8), false);
         begin += b.count;
         p->buckets.push_back(std::move(b));
@@ -1122,7 +1143,7 @@ int gputils_gels_ragged_plan_tune(gputils_gels_plan_t plan, const double *A, con
                     }
                     rc = qr::launch_ragged(bk.maxe, bk.method, bk.waves, bk.grid, st, plan->d_items,
                                            plan->d_wstart + bk.wbase, A, scratch, refine_steps,
-                                           bk.queue ? plan->d_queue + 2 * bi : nullptr);
+                                           bk.queue ? plan->d_queue + 2 * bi : nullptr, plan->cus);
                     if (rc != GPUTILS_OK) break;
                     e = hipEventRecord(ev1, st);
                     if (e == hipSuccess) e = hipEventSynchronize(ev1);
