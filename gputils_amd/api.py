@@ -35,9 +35,15 @@ def to_matrices(t: torch.Tensor) -> torch.Tensor:
     return t.transpose(-1, -2)
 
 
+# the handle itself, where this torch has the (private) call for it:
+# torch.cuda.current_stream() builds a Stream object around it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle() -> int:
-    # the handle itself: torch.cuda.current_stream() builds a Stream object around it
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t):
