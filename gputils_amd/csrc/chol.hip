@@ -1090,11 +1090,16 @@ int potrs_large(int64_t n, int64_t nrhs, const T *L, int64_t lda, int64_t stride
     const int64_t nb = ceil_div(n, 16);
     if (n <= kStripMaxN) {
         // at most 108 KB of LDS (n = kStripMaxN in FP64)
-        const size_t lds = sizeof(T) * (size_t)(256 * nb + 16 * nb * kRhsChunk + 16 * kRhsChunk);
+        auto bytes = [](int64_t blocks) {
+            return sizeof(T) * (size_t)(256 * blocks + 16 * blocks * kRhsChunk + 16 * kRhsChunk);
+        };
+        const size_t lds = bytes(nb);
         auto kern = n <= kStripThreads ? potrs_strips_kernel<T, 1> : potrs_strips_kernel<T, 2>;
+        // the same value from every call: another thread's launch of this kernel
+        // may come between this line and the next
         if (lds > 64 * 1024)
             GPUTILS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes(kStripMaxN / 16)));
         hipLaunchKernelGGL(kern, dim3((unsigned)batch), dim3(kStripThreads), lds, st, (int)n, (int)nrhs, L, lda,
                            strideL, B, ldb, strideB, info, batch, skip);
         return launch_check("potrs_strips_kernel");

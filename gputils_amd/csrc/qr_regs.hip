@@ -536,7 +536,7 @@ struct QrPick {
     }
 };
 
-constexpr int kMaxLds = 160 * 1024;
+constexpr int kMaxDyn = 128 * 1024;  // of 160 KB; the kernels' own arrays take 17 at most
 // From here on one workgroup per tall matrix keeps half the CUs busy, and the
 // panel form's extra passes over the matrix cost more than they spread.
 constexpr int64_t kWholeBatch = 128;
@@ -578,10 +578,12 @@ int gels(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t strideA,
     // one launch where R and the right-hand sides fit the LDS
     const QrPick<T> whole(m, n + nrhs, batch >= kWholeBatch);
     const size_t dyn = nrhs > 0 ? sizeof(T) * (size_t)((n | 1) * (n + nrhs)) : 0;
-    if (whole.kern != nullptr && n <= 2 * kWave && whole.lds + (int64_t)dyn <= kMaxLds) {
+    if (whole.kern != nullptr && n <= 2 * kWave && dyn <= (size_t)kMaxDyn) {
+        // the same value from every call: another thread's launch of this kernel
+        // may come between this line and the next
         if (whole.lds + dyn > 64 * 1024)
             GPUTILS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(whole.kern),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn));
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, kMaxDyn));
         hipLaunchKernelGGL(whole.kern, dim3((unsigned)batch), dim3(whole.threads), dyn, st, (int)m, (int)n, (int)nrhs,
                            A, lda, strideA, B, ldb, strideB, (T *)nullptr, (int64_t)0, info, batch);
         return launch_check("qr_regs_kernel");
