@@ -2,7 +2,7 @@
 // the QR / least-squares and SVD kernels (LAPACK dlarfg / dlarf conventions:
 // beta = -sign(alpha)*||[alpha; x]||, tau = (beta - alpha)/beta,
 // v = [1; x / (alpha - beta)]).  The factorisation spreads the columns over
-// the workgroup's wavefronts (four unless a kernel asks for another count).
+// the workgroup's four wavefronts.
 #pragma once
 
 #include "common.hpp"
@@ -174,15 +174,15 @@ __device__ __forceinline__ T row16_sum(T x) {
     return row16_plus<0x140>(x);  // row_mirror
 }
 
-// x_c <- (I - tau v v^T) x_c for the columns c = c0, c0 + NW, ... < n (the
-// columns one of NW wavefronts owns), v = [1; A[j+1:m, j]], for
+// x_c <- (I - tau v v^T) x_c for the columns c = c0, c0 + kWaves, ... < n (the
+// columns one wavefront owns), v = [1; A[j+1:m, j]], for
 // m - j - 1 <= 16 KR: each 16-lane group of the wavefront takes one column
 // (four at a time), lane l of a group rows j + 1 + l + 16 k (k < KR, v held
 // in registers for all the columns), and reduces its dot product within
 // its 16 lanes.  Four columns then cost one set of row loads and one
 // four-step reduction, where the 64-lane form below pays a six-step
 // reduction per column.
-template <typename T, typename DOT, int NW, int KR>
+template <typename T, typename DOT, int KR>
 __device__ __forceinline__ void apply_reflector_cols16(T *A, int64_t lda, int m, int j, T tau, int c0, int n) {
     const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
     const T *v = A + (int64_t)j * lda;
@@ -197,8 +197,8 @@ __device__ __forceinline__ void apply_reflector_cols16(T *A, int64_t lda, int m,
             vr[k] = (i < m) ? e : T(0);
         }
     }
-    for (int cq = c0; cq < n; cq += 4 * NW) {
-        const int c = cq + NW * g;
+    for (int cq = c0; cq < n; cq += 4 * kWaves) {
+        const int c = cq + kWaves * g;
         const bool ok = c < n;
         T *x = A + (int64_t)(ok ? c : cq) * lda;
         T xr[KR];
@@ -227,22 +227,22 @@ __device__ __forceinline__ void apply_reflector_cols16(T *A, int64_t lda, int m,
     // the caller's barrier orders these writes before other wavefronts' reads
 }
 
-// x_c <- (I - tau v v^T) x_c for the columns c = c0, c0 + NW, ... < n (the
-// columns one of NW wavefronts owns), v = [1; A[j+1:m, j]], four columns at a
+// x_c <- (I - tau v v^T) x_c for the columns c = c0, c0 + kWaves, ... < n (the
+// columns one wavefront owns), v = [1; A[j+1:m, j]], four columns at a
 // time: their dot products are accumulated together and their reductions
 // overlap, so the wavefront waits for one set of reductions per four
 // columns instead of one per column.  Past the last column the slots work
 // on the first owned column with tau w = 0.
-template <typename T, typename DOT, int NW = kWaves>
+template <typename T, typename DOT>
 __device__ __forceinline__ void apply_reflector_cols(T *A, int64_t lda, int m, int j, T tau, int c0, int n) {
     const int lane = threadIdx.x & 63;
     const T *v = A + (int64_t)j * lda;
-    for (int cq = c0; cq < n; cq += 4 * NW) {
+    for (int cq = c0; cq < n; cq += 4 * kWaves) {
         T *x[4];
         bool ok[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int c = cq + NW * q;
+            const int c = cq + kWaves * q;
             ok[q] = c < n;
             x[q] = A + (int64_t)(ok[q] ? c : cq) * lda;
         }
@@ -275,19 +275,13 @@ __device__ __forceinline__ void apply_reflector_cols(T *A, int64_t lda, int m, i
 
 // Householder QR of the m x n (m >= n) matrix at A (LDS or global), tau[j]
 // for j < n, column norms accumulated in ACC and the reflectors' dot
-// products in DOT.  s_tau: two LDS slots.  Ends with a barrier.  Columns n ..
-// ntot-1 (stored after the factorised ones) receive every reflector
-// without being factorised: a right-hand side stored there ends as Q^T b.
-// NW (a power of two) wavefronts: column c is owned by wavefront c % NW.
-// Each column's arithmetic is the same for every NW.  KR16 != 0 applies the
-// reflectors with 16-lane groups (apply_reflector_cols16; KR16 > 0 requires
-// m <= 16 KR16 + 1).
-template <typename T, typename ACC, typename DOT = ACC, int NW = kWaves, int KR16 = 0>
-__device__ __forceinline__ void hqr_factor(T *A, int64_t lda, int m, int n, T *tau, T *s_tau, int ntot = 0) {
-    static_assert(NW >= 1 && (NW & (NW - 1)) == 0, "NW must be a power of two");
+// products in DOT.  s_tau: two LDS slots.  Ends with a barrier.  Column c is
+// owned by wavefront c % kWaves.  KR16 > 0 applies the reflectors with 16-lane
+// groups (apply_reflector_cols16; m <= 16 KR16 + 1).
+template <typename T, typename ACC, typename DOT = ACC, int KR16 = 0>
+__device__ __forceinline__ void hqr_factor(T *A, int64_t lda, int m, int n, T *tau, T *s_tau) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (n <= 0) return;
-    if (ntot < n) ntot = n;
     if (wave == 0) {
         const T t = make_reflector<T, ACC>(A, lda, m, 0);
         if (lane == 0) {
@@ -298,8 +292,8 @@ __device__ __forceinline__ void hqr_factor(T *A, int64_t lda, int m, int n, T *t
     __syncthreads();
     for (int j = 0; j < n; ++j) {
         const T t = s_tau[j & 1];
-        if (j + 1 < ntot && wave == ((j + 1) & (NW - 1))) {
-            if (j + 1 < n && m <= 8 * kWave) {
+        if (j + 1 < n && wave == ((j + 1) & (kWaves - 1))) {
+            if (m <= 8 * kWave) {
                 // as many row groups as the column has (the terms past m
                 // are zeros either way)
                 const T t1 = (m <= 2 * kWave)   ? update_and_reflect<T, ACC, DOT, 2>(A, lda, m, j, t)
@@ -311,19 +305,17 @@ __device__ __forceinline__ void hqr_factor(T *A, int64_t lda, int m, int n, T *t
                 }
             } else {
                 apply_reflector_col<T, DOT>(A, lda, m, j, t, j + 1);
-                if (j + 1 < n) {
-                    const T t1 = make_reflector<T, ACC>(A, lda, m, j + 1);
-                    if (lane == 0) {
-                        s_tau[(j + 1) & 1] = t1;
-                        tau[j + 1] = t1;
-                    }
+                const T t1 = make_reflector<T, ACC>(A, lda, m, j + 1);
+                if (lane == 0) {
+                    s_tau[(j + 1) & 1] = t1;
+                    tau[j + 1] = t1;
                 }
             }
         }
         if (t != T(0)) {
-            const int c0 = j + 2 + ((wave - (j + 2)) & (NW - 1));
-            if constexpr (KR16 != 0) apply_reflector_cols16<T, DOT, NW, KR16>(A, lda, m, j, t, c0, ntot);
-            else apply_reflector_cols<T, DOT, NW>(A, lda, m, j, t, c0, ntot);
+            const int c0 = j + 2 + ((wave - (j + 2)) & (kWaves - 1));
+            if constexpr (KR16 != 0) apply_reflector_cols16<T, DOT, KR16>(A, lda, m, j, t, c0, n);
+            else apply_reflector_cols<T, DOT>(A, lda, m, j, t, c0, n);
         }
         __syncthreads();
     }

@@ -48,7 +48,7 @@ struct Acc<double> {
 template <typename T, int MAXE>
 __global__ __launch_bounds__(kThreads) void gels_kernel(int m, int n, int nrhs, T *A, int64_t lda,
                                                         int64_t strideA, T *B, int64_t ldb,
-                                                        int64_t strideB, T *tauws, int *info,
+                                                        int64_t strideB, int *info,
                                                         int64_t batch) {
     using ACC = typename Acc<T>::type;
     constexpr int kLds = MAXE > 0 ? MAXE : 1;
@@ -83,8 +83,6 @@ __global__ __launch_bounds__(kThreads) void gels_kernel(int m, int n, int nrhs, 
         __syncthreads();
         for (int i = threadIdx.x; i < n; i += kThreads) bb[i + (int64_t)r * ldb] = c[i];
     }
-    if (tauws != nullptr)
-        for (int i = threadIdx.x; i < n; i += kThreads) tauws[b * n + i] = tau[i];
     if (threadIdx.x == 0 && info != nullptr) info[b] = 0;
 }
 
@@ -696,7 +694,7 @@ int launch_ragged(int maxe, int method, int waves, int grid, hipStream_t st, con
 
 template <typename T>
 int gels_dispatch(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t strideA, T *B,
-                  int64_t ldb, int64_t strideB, T *tauws, int *info, int64_t batch, hipStream_t st) {
+                  int64_t ldb, int64_t strideB, int *info, int64_t batch, hipStream_t st) {
     if (m <= qrr::kMaxRows && n <= qrr::kMaxTri)
         return qrr::gels<T>(m, n, nrhs, A, lda, strideA, B, ldb, strideB, info, batch, st);
     const size_t dyn = sizeof(T) * (size_t)(n + m);
@@ -708,7 +706,7 @@ int gels_dispatch(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t
     const int64_t mn = m * n;
 #define GPUTILS_GELS(ME)                                                                                  \
     hipLaunchKernelGGL((gels_kernel<T, ME>), grid, block, dyn, st, (int)m, (int)n, (int)nrhs, A, lda, strideA, \
-                       B, ldb, strideB, tauws, info, batch)
+                       B, ldb, strideB, info, batch)
     constexpr int kBig = (int)(56 * 1024 / sizeof(T));
     if (mn <= 4096) GPUTILS_GELS(4096);
     else if (mn <= kBig) GPUTILS_GELS(kBig);
@@ -892,7 +890,7 @@ int gputils_sgels_batched(int64_t m, int64_t n, int64_t nrhs, float *A, int64_t 
     if (m == 0 || n == 0 || batch == 0) return GPUTILS_OK;
     GPUTILS_ARG(A != nullptr, 4, "A is NULL");
     GPUTILS_ARG(nrhs == 0 || B != nullptr, 7, "B is NULL");
-    return qr::gels_dispatch<float>(m, n, nrhs, A, lda, strideA, B, ldb, strideB, nullptr, info, batch,
+    return qr::gels_dispatch<float>(m, n, nrhs, A, lda, strideA, B, ldb, strideB, info, batch,
                                     as_stream(stream));
 }
 
@@ -907,7 +905,7 @@ int gputils_dgels_batched(int64_t m, int64_t n, int64_t nrhs, double *A, int64_t
     if (m == 0 || n == 0 || batch == 0) return GPUTILS_OK;
     GPUTILS_ARG(A != nullptr, 4, "A is NULL");
     GPUTILS_ARG(nrhs == 0 || B != nullptr, 7, "B is NULL");
-    return qr::gels_dispatch<double>(m, n, nrhs, A, lda, strideA, B, ldb, strideB, nullptr, info, batch,
+    return qr::gels_dispatch<double>(m, n, nrhs, A, lda, strideA, B, ldb, strideB, info, batch,
                                      as_stream(stream));
 }
 

@@ -512,7 +512,9 @@ struct QrPick {
         else if (nt <= 48) set<16, 4, KR, 3>();
         else if (nt <= 64) set<16, 8, KR, 2>();
         else if (nt <= 96) set<16, 8, KR, 3>();
-        else if (nt <= 128 && (int)sizeof(T) * KR < 128) set<16, 16, KR, 2>();
+        else if constexpr ((int)sizeof(T) * KR < 128) {
+            if (nt <= 128) set<16, 16, KR, 2>();
+        }
     }
     // whole: as many columns as fit one workgroup; else a panel of kPanel
     QrPick(int64_t m, int64_t nt, bool whole) {
@@ -523,15 +525,16 @@ struct QrPick {
         else if (m <= 256) set16<16>((int)nt);
         if (kern != nullptr) return;
         if (nt <= kPanel) {
-            if (m <= 256) set<64, 16, 4, 1>();
-            else if (m <= 384) set<64, 16, 6, 1>();
+            if (m <= 384) set<64, 16, 6, 1>();
             else if (m <= 640) set<64, 16, 10, 1>();
             else if (m <= kMaxRows) set<64, 16, 16, 1>();
         } else if (whole) {
             constexpr int k8 = 8 / (int)sizeof(T);  // twice the slots in FP32
             if (m <= 384 && nt <= 80 * k8) set<64, 16, 6, 5 * k8>();
             else if (m <= 640 && nt <= 48 * k8) set<64, 16, 10, 3 * k8>();
-            else if (sizeof(T) == 4 && m <= kMaxRows && nt <= 64) set<64, 16, 16, 4>();
+            else if constexpr (sizeof(T) == 4) {
+                if (m <= kMaxRows && nt <= 64) set<64, 16, 16, 4>();
+            }
         }
     }
 };
