@@ -121,6 +121,14 @@ __device__ __forceinline__ void mark_tails(T *A, int64_t lda, int m, int n, cons
     }
 }
 
+// Wavefronts per SIMD to leave registers for: what the column steps alone take,
+// by the 32-bit words of the columns.  Left to itself the compiler gives the
+// rare path below some more, and 8192 FP32 100 x 30 factorisations (66 registers
+// where 64 fit) take 153 us instead of 147.
+constexpr int qr_waves(int words) {
+    return words <= 14 ? 8 : words <= 16 ? 7 : words <= 20 ? 6 : words <= 24 ? 5 : words <= 32 ? 4 : words <= 48 ? 3 : words <= 64 ? 2 : 1;
+}
+
 // QR of one matrix per workgroup, and with nrhs > 0 the least-squares
 // solution: the right-hand sides ride along as columns n .. n + nrhs - 1, so
 // the factorisation leaves Q^T b; R and those go to LDS and one wavefront
@@ -129,13 +137,6 @@ __device__ __forceinline__ void mark_tails(T *A, int64_t lda, int m, int n, cons
 // infinities and NaNs reach rows that the reflector does not.  A column that
 // has met one is NaN throughout and so is its scalar: the matrix, still as it
 // was in memory, is then factorised again there (hh::hqr_plain).
-// Wavefronts per SIMD to leave registers for: what the column steps alone take,
-// by the 32-bit words of the columns.  Left to itself the compiler gives the
-// rare path above some more, and 8192 FP32 100 x 30 factorisations (66 registers
-// where 64 fit) take 153 us instead of 147.
-constexpr int qr_waves(int words) {
-    return words <= 14 ? 8 : words <= 16 ? 7 : words <= 20 ? 6 : words <= 24 ? 5 : words <= 32 ? 4 : words <= 48 ? 3 : words <= 64 ? 2 : 1;
-}
 template <typename T, int LPC, int NW, int KR, int SL>
 __global__ __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(
     qr_waves(KR *SL *(int)sizeof(T) / 4) > NW / 4 ? qr_waves(KR *SL *(int)sizeof(T) / 4) : (NW + 3) / 4))) void qr_regs_kernel(int m, int n, int nrhs, T *A, int64_t lda,
@@ -490,9 +491,12 @@ namespace {
 constexpr int kPanel = 16;
 
 // The instantiation for m rows and nt columns, or NULL.  16-lane columns up
-// to 256 rows and 128 columns; taller or wider ones by whole wavefronts, as
-// many slots as 128 registers a lane hold (16 wavefronts on one CU).  Every
-// m <= kMaxRows takes kPanel columns.
+// to 256 rows and 128 columns (FP64 of more than 160 rows: 96, where the
+// registers end); taller matrices by whole wavefronts, kPanel columns of them,
+// which every m <= kMaxRows takes, and whatever is wider in panels.  Several
+// slots of whole wavefronts spilled 13 to 100 registers and were 2 to 5 times
+// slower than panels for any batch: 128 and 1024 FP32 384 x 80 factorisations
+// 281 and 1259 us, in panels 104 and 303.
 template <typename T>
 struct QrPick {
     void (*kern)(int, int, int, T *, int64_t, int64_t, T *, int64_t, int64_t, T *, int64_t, int *, int64_t) = nullptr;
@@ -516,42 +520,28 @@ struct QrPick {
             if (nt <= 128) set<16, 16, KR, 2>();
         }
     }
-    // whole: as many columns as fit one workgroup; else a panel of kPanel
-    QrPick(int64_t m, int64_t nt, bool whole) {
+    QrPick(int64_t m, int64_t nt) {
         if (m <= 32) set16<2>((int)nt);
         else if (m <= 64) set16<4>((int)nt);
         else if (m <= 112) set16<7>((int)nt);
         else if (m <= 160) set16<10>((int)nt);
         else if (m <= 256) set16<16>((int)nt);
-        if (kern != nullptr) return;
-        if (nt <= kPanel) {
+        else if (nt <= kPanel) {
             if (m <= 384) set<64, 16, 6, 1>();
             else if (m <= 640) set<64, 16, 10, 1>();
             else if (m <= kMaxRows) set<64, 16, 16, 1>();
-        } else if (whole) {
-            constexpr int k8 = 8 / (int)sizeof(T);  // twice the slots in FP32
-            if (m <= 384 && nt <= 80 * k8) set<64, 16, 6, 5 * k8>();
-            else if (m <= 640 && nt <= 48 * k8) set<64, 16, 10, 3 * k8>();
-            else if constexpr (sizeof(T) == 4) {
-                if (m <= kMaxRows && nt <= 64) set<64, 16, 16, 4>();
-            }
         }
     }
 };
 
 constexpr int kMaxDyn = 128 * 1024;  // of 160 KB; the kernels' own arrays take 17 at most
-// From here on one workgroup per tall matrix keeps half the CUs busy, and the
-// panel form's extra passes over the matrix cost more than they spread.
-constexpr int64_t kWholeBatch = 128;
 
 }  // namespace
 
 template <typename T>
 int geqrf(int64_t m, int64_t n, T *A, int64_t lda, int64_t strideA, T *tau, int64_t strideTau, int *info,
           int64_t batch, hipStream_t st) {
-    // taller matrices in one workgroup each only where the batch fills the
-    // chip that way; panels spread the updates of a few matrices over it
-    const QrPick<T> whole(m, n, batch >= kWholeBatch);
+    const QrPick<T> whole(m, n);
     if (whole.kern != nullptr) {
         hipLaunchKernelGGL(whole.kern, dim3((unsigned)batch), dim3(whole.threads), 0, st, (int)m, (int)n, 0, A, lda,
                            strideA, A, lda, strideA, tau, strideTau, info, batch);
@@ -563,7 +553,7 @@ int geqrf(int64_t m, int64_t n, T *A, int64_t lda, int64_t strideA, T *tau, int6
     for (int64_t j = 0; j < n; j += kPanel) {
         const int64_t w = std::min<int64_t>(kPanel, n - j), rest = n - j - w;
         T *p = A + j + j * lda;
-        const QrPick<T> panel(m - j, w, false);
+        const QrPick<T> panel(m - j, w);
         hipLaunchKernelGGL(panel.kern, dim3((unsigned)batch), dim3(panel.threads), 0, st, (int)(m - j), (int)w, 0, p,
                            lda, strideA, p, lda, strideA, tau != nullptr ? tau + j : tau, strideTau, info, batch);
         int rc = launch_check("qr_regs_kernel");
@@ -579,7 +569,7 @@ template <typename T>
 int gels(int64_t m, int64_t n, int64_t nrhs, T *A, int64_t lda, int64_t strideA, T *B, int64_t ldb, int64_t strideB,
          int *info, int64_t batch, hipStream_t st) {
     // one launch where R and the right-hand sides fit the LDS
-    const QrPick<T> whole(m, n + nrhs, batch >= kWholeBatch);
+    const QrPick<T> whole(m, n + nrhs);
     const size_t dyn = nrhs > 0 ? sizeof(T) * (size_t)((n | 1) * (n + nrhs)) : 0;
     if (whole.kern != nullptr && n <= 2 * kWave && dyn <= (size_t)kMaxDyn) {
         // the same value from every call: another thread's launch of this kernel

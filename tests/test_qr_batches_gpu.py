@@ -1,6 +1,6 @@
-"""QR, least squares and Q application in the forms that batches take: tall
-matrices in one workgroup each (from 128 matrices on), at the widest that its
-registers hold and one column more, and ormqr with four columns a wavefront.
+"""QR, least squares and Q application of batches: 130 tall matrices at the
+rows where the kernels change and around multiples of a panel's columns, and
+ormqr with four columns a wavefront.
 
 Two different matrices, repeated over the batch; every copy has to come out
 the same, and the two agree with numpy in 64 bits (Gaussian, m >= 1.3 n, so to
@@ -58,6 +58,20 @@ def test_tall_batches(m, n, dtype):
         ref = np.linalg.lstsq(A[i][:, :n - 3], B[i], rcond=None)[0]
         assert np.abs(X[i][:n - 3] - ref).max() <= tol(dtype) * np.abs(ref).max()
     assert torch.equal(b[:, :, n - 3:], was[:, :, n - 3:])
+
+
+@pytest.mark.parametrize("m,n", [(257, 17), (300, 40), (1000, 33)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_results_do_not_depend_on_the_batch(m, n, dtype):
+    """Factors and solutions of the first matrices of 200, and of these alone: bit for bit."""
+    r = np.random.default_rng(m * n)
+    A, B = (torch.from_numpy(r.standard_normal(s)).to(dtype).cuda() for s in ((200, n, m), (200, 2, m)))
+    for k in (1, 100):
+        for fn in (lambda a, b: api.geqrf_batched(a), api.gels_batched):
+            a, b, a1, b1 = A.clone(), B.clone(), A[:k].clone(), B[:k].clone()
+            fn(a, b)
+            fn(a1, b1)
+            assert torch.equal(a[:k], a1) and torch.equal(b[:k], b1)
 
 
 # one to ten registers a column; more than 64 reflectors where there are rows for them
