@@ -629,7 +629,7 @@ __global__ __launch_bounds__(kThreads) void posv_kernel(int n, int nrhs, T *A, i
 // this one 70 us.
 constexpr int kStripThreads = 512;
 constexpr int kStripWorkers = kStripThreads / kWave - 1;
-constexpr int kStripSlots = 6;  // strips per wavefront: more spill the FP64 accumulators
+constexpr int kStripSlots = 6;  // strips per wavefront; FP64 has 31 registers in scratch here already
 constexpr int64_t kStripMaxN = 16 * kStripWorkers * kStripSlots;
 static_assert(kStripMaxN <= 2 * kStripThreads, "potrs_strips_kernel holds two rows a thread");
 constexpr int64_t kStripMaxLd = 1 << 26;  // lane offsets of up to 13 columns are 32-bit
@@ -828,7 +828,7 @@ __device__ __forceinline__ void substitute(int n, int nrhs, const T *l, int64_t 
 // (rows along the lanes, so L is read contiguously), two barriers per step.
 // 256 systems of n = 200 in FP64, one right-hand side: 310 us for the
 // substitution by columns with two barriers and a tree reduction each,
-// 47 us now.
+// 49 us now.
 // skip != nullptr: systems with skip[b] != 0 (a failed factorisation) are
 // left as they are, as LAPACK dposv leaves B.
 // A factor with a diagonal entry that has no normal reciprocal is substituted

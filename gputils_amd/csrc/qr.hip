@@ -507,7 +507,7 @@ constexpr int ragged_waves(int maxe, int nw, int method, bool many) {
 // 0 is bound by the chain of the reflector (about 1350 cycles for short
 // columns) and for tall ones by issue; with A streamed from LDS for every
 // column it took 3700 to 5300.  4096 systems of the configuration, one
-// refinement step: default shapes 1533 -> 1071 us, tuned 1119 -> 855 us.  The plan
+// refinement step: default shapes 1533 -> 1030 us, tuned 1119 -> 817 us.  The plan
 // picks METHOD, NW and the grid per bucket.  For one METHOD every system's
 // arithmetic is the same for every NW and every item-to-workgroup
 // assignment, so the results are too; the two methods round the FP32

@@ -7,9 +7,10 @@
 // the lanes that own it, and only the reflector goes through LDS.  What
 // bounds a step now is the chain reflector -> dot product -> update -> next
 // reflector (about 0.6 us in FP32, 1 us in FP64) and, with many matrices,
-// instruction issue.  Before -> now: least squares of 1024 FP32 100 x 30
-// systems 91 -> 33 us, of 8192 402 -> 144 us; QR of one FP64 600 x 150 matrix
-// 6320 -> 250 us, its 150 columns of Q 10357 -> 63 us.
+// instruction issue (VALU issue in 65 % of the cycles of 1024 least-squares
+// systems).  Before -> now: least squares of 1024 FP32 100 x 30 systems 91 -> 35
+// us; QR of one FP64 600 x 150 matrix 6320 -> 250 us, its 150 columns of Q
+// 10357 -> 64 us.
 #include <algorithm>
 
 #include "qr_regs.hpp"
@@ -254,7 +255,7 @@ __global__ __launch_bounds__(kOrmThreads) void ormqr_regs_kernel(int trans, int 
     // The rows of a chunk's unit entries lie in one block of 64: it and block 0
     // change places in the registers and in V, so that the unit entry is always
     // in slot 0.  Its product joins the dot product after the reduction (see
-    // RegQr).  A 600 x 150 FP64 QR, solution and Q take 405 us so, as with the
+    // RegQr).  A 600 x 150 FP64 QR, solution and Q took 405 us so, as with the
     // entry in the lanes' sums, and 458 with the row's register selected in
     // every step.
     int head = 0;  // block in slot 0
@@ -593,7 +594,7 @@ int ormqr(int trans, int64_t m, int64_t mout, int64_t ncols, int64_t k, const T 
           const T *tau, int64_t strideTau, T *C, int64_t ldc, int64_t strideC, int64_t batch, hipStream_t st) {
     // four columns a wavefront once that still gives four wavefronts per SIMD:
     // below it the chain of each reflector is what counts (1024 FP32 100 x 30
-    // factors, 30 columns: 34 us, 189 with the column in LDS)
+    // factors, 30 columns: 40 us, 189 with the column in LDS)
     const bool wide = ncols * batch >= 4 * 4096 && m <= 640;
     const int64_t per = (wide ? 4 : 1) * kOrmWaves;
     for (int64_t c0 = 0; c0 < ncols; c0 += per * 65535) {
