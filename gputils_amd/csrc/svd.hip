@@ -706,14 +706,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         if (gl == 0) sig[j] = sqrt(s);
     }
     __syncthreads();
+    // Descending, ties by index.  The places must be a permutation for every
+    // input, as ord indexes X and W below and an entry that nobody wrote
+    // would lead anywhere: so the order is that of the bits without the
+    // sign, total also with NaN (first, above Inf) and the same as that of
+    // the values for all others, which are not negative.
+    auto key = [](double s) { return __builtin_bit_cast(int64_t, s) & INT64_MAX; };
     for (int j = tid; j < n; j += kThreads) {
         const double sj = sig[j];
+        const int64_t kj = key(sj);
         double smax = 0.0;
         int ps = 0;
         for (int k = 0; k < n; ++k) {
             const double sk = sig[k];
+            const int64_t kk = key(sk);
             smax = sk > smax ? sk : smax;
-            ps += (sk > sj || (sk == sj && k < j)) ? 1 : 0;
+            ps += (kk > kj || (kk == kj && k < j)) ? 1 : 0;
         }
         pos[j] = ps;
         ord[ps] = j;
